@@ -219,10 +219,8 @@ def _rows(case):
 
 
 def work(case):
-    """Bytes and operations of one pass. A model's state stays on the chip as far as it fits,
-    so the bytes are its tables once and its recorded rows once; a network's synapse state
-    does not fit on the chip and is read and written once a window of its shortest delay (38
-    steps). Operations: about 150 a gate variable and step (two rates of one exponential each
+    """Bytes and operations of one pass. A model's state can stay on the chip for the run, so the bytes are its tables once and its recorded rows once (about 60 a compartment, 30 a
+    synapse). Operations: about 150 a gate variable and step (two rates of one exponential each
     and the update), 30 a compartment and step (currents, membrane update, elimination and
     substitution), 20 a synapse and step; a gradient costs three forward passes."""
     rows, kind, n = _rows(case), case["kind"], case["cells"]
@@ -236,8 +234,7 @@ def work(case):
         return dict(bytes=comps * 60.0 + 4.0 * n * rows, flops=rows * (gates * gate + comps * comp_ops))
     if kind == "net":
         syn = n * case["degree"]
-        windows = math.ceil(rows / 38)
-        return dict(bytes=windows * syn * 20.0 + 4.0 * rows * min(n, 100),
+        return dict(bytes=n * 100.0 + syn * 30.0 + 4.0 * rows * min(n, 100),
                     flops=rows * (syn * syn_ops + n * (3 * gate + comp_ops)))
     if kind == "mixed":
         comps = n * 127.0
