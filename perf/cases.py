@@ -219,7 +219,8 @@ def _rows(case):
 
 
 def work(case):
-    """Bytes and operations of one pass. A model's state can stay on the chip for the run, so the bytes are its tables once and its recorded rows once (about 60 a compartment, 30 a
+    """Bytes and operations of one pass. A model's state can stay on the chip for the run, so
+    the bytes are its tables once and its recorded rows once (about 60 a compartment, 30 a
     synapse). Operations: about 150 a gate variable and step (two rates of one exponential each
     and the update), 30 a compartment and step (currents, membrane update, elimination and
     substitution), 20 a synapse and step; a gradient costs three forward passes."""
