@@ -21,7 +21,7 @@ __device__ __forceinline__ uint64_t mix64(uint64_t x) {
 }
 
 // operand i of pair k: raw random bits, or (every other pair) a random significand and sign
-// with an exponent drawn from [80, 175], around the fast path's range [87, 167]
+// with an exponent drawn from [80, 175], inside div_rn's fast range [67, 187]
 __device__ __forceinline__ float operand(uint64_t seed, uint64_t k, int i) {
     const uint64_t h = mix64(seed ^ mix64(2 * k + (uint64_t)i));
     uint32_t bits = (uint32_t)h;

@@ -48,6 +48,34 @@ bool const_below_root(const edenhip_model_desc *d, int64_t c0, int32_t n) {
     return true;
 }
 
+// Voltages at which gate_next_fast's divisions stay inside the normal floats: rate parameters of
+// moderate size (any other gate gets the empty range, so the general path), and a voltage within
+// 24 scales of each midpoint. The exponentials are then within 2^+-35, every rate within
+// 2^-63 .. 2^58 (or zero), inf above 2^-121 and the time factor within 2^+-84. HH squid rates
+// (scale 10 around -40 mV): -279 .. 173 mV.
+void gate_safe_range(DGate &G, float dt) {
+    G.ras = 1.0 / (double)G.as;
+    G.rbs = 1.0 / (double)G.bs;
+    G.vlo = 1.0f;
+    G.vhi = -1.0f;
+    float lo = -FLT_MAX, hi = FLT_MAX;
+    const bool tau_inf = (G.forms & 0xF0) != 0;
+    auto moderate = [](float x, float a, float b) { return x >= a && x <= b; };
+    auto rate = [&](int form, float r, float mid, float scale, bool zero_ok) {
+        if (form == RATE_LEMS || !(moderate(r, 0x1p-28f, 0x1p22f) || (zero_ok && r == 0.0f))) return false;
+        if (form == RATE_FIXED) return true;
+        const float s = std::fabs(scale);
+        if (!moderate(s, 0x1p-20f, 0x1p20f) || !(std::fabs(mid) < 0x1p20f)) return false;
+        lo = std::max(lo, mid - 23.9f * s);
+        hi = std::min(hi, mid + 23.9f * s);
+        return true;
+    };
+    if (!moderate(dt * G.q10, 0x1p-20f, 0x1p20f)) return;
+    if (!rate(G.forms & 0xF, G.ar, G.am, G.as, !tau_inf) || !rate((G.forms >> 8) & 0xFF, G.br, G.bm, G.bs, true)) return;
+    G.vlo = lo;
+    G.vhi = hi;
+}
+
 struct Bucket {
     int tpb = 64;
     bool split = false;   // one extra wave runs the channel phase concurrently
@@ -488,6 +516,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
             G.q10 = g.q10;
             G.ar = g.alpha.rate; G.am = g.alpha.midpoint; G.as = g.alpha.scale;
             G.br = g.beta.rate; G.bm = g.beta.midpoint; G.bs = g.beta.scale;
+            gate_safe_range(G, d->dt);
         }
     }
     ctx->n_gates = (int)gates.size();
