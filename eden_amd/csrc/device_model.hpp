@@ -361,19 +361,23 @@ __device__ __forceinline__ bool gate_next_fast(const DGate &G, float V, float q,
     const float blend = (float)exp_taylor((double)(-fminf(tau_factor, 200.0f)));
     float nv = (blend) * q + (1.0f - blend) * inf;
     const bool ok = (V >= G.vlo) & (V <= G.vhi) & (nv == nv) & (inf == inf);
-    if (!(nv > 1e-6f)) nv = 1e-6f;
-    if (!(nv < (float)(1 - 1e-6))) nv = (float)(1 - 1e-6);
+    nv = fminf(fmaxf(nv, 1e-6f), (float)(1 - 1e-6));
     out = init ? inf : nv;
     return ok;
 }
 
-__device__ __forceinline__ float gate_next(const DGate &G, float V, float q, bool init, float dt) {
+// G: the gate's values (in registers), table: its table entry, read where the divisions are the
+// compiler's
+__device__ __forceinline__ float gate_next(const DGate &G, const DGate *table, float V, float q, bool init, float dt) {
     float nv;
     if (__builtin_expect(!gate_next_fast(G, V, q, init, dt, nv), 0)) {
         DivIeee d;
-        nv = gate_next_t(d, G, V, q, init, dt);
+        nv = gate_next_t(d, *table, V, q, init, dt);
     }
     return nv;
+}
+__device__ __forceinline__ float gate_next(const DGate &G, float V, float q, bool init, float dt) {
+    return gate_next(G, &G, V, q, init, dt);
 }
 
 // Thomas Wang's 64-bit integer hash (published 1997); EDEN's RNG mixer
@@ -555,6 +559,133 @@ __device__ __forceinline__ void channels_step(const DGate *__restrict__ gates, c
         }
     }
 }
+
+// Voltage of a one-compartment cell after a step (eden/Eden.cpp:6057-6107): the semi-implicit
+// update, no elimination, the root's divide; rC = 1 / C in double (div_c).
+__device__ __forceinline__ float point_update(float V, float I_int, float G_int, float invrc, double rC, float dt) {
+    float D = 1 * div_c(G_int, rC) + invrc;
+    const float x = V + div_c(dt * (I_int + ((V * G_int))), rC);
+    D = 1 + D * dt;
+    return div_rn(x, D);
+}
+
+// x of lane L of the quad, in all four of its lanes
+template <int L>
+__device__ __forceinline__ float quad_bcast(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), L * 0x55, 0xF, 0xF, true));
+}
+
+// (I, G) + the quad's four values of (i, g) in lane order, the two chains side by side (a DPP
+// operand may not be read within two instructions of the write of any operand it goes with)
+__device__ __forceinline__ void quad_add2(float &I, float &G, float i, float g) {
+    I = I + quad_bcast<0>(i);
+    G = G + quad_bcast<0>(g);
+    I = I + quad_bcast<1>(i);
+    G = G + quad_bcast<1>(g);
+    I = I + quad_bcast<2>(i);
+    G = G + quad_bcast<2>(g);
+    I = I + quad_bcast<3>(i);
+    G = G + quad_bcast<3>(g);
+}
+
+// Channels of a one-compartment cell on the four lanes of a quad: lane s holds channel s's
+// density and gate variable s. A channel's open fraction multiplies its gates' values in order,
+// each `instances` times (channels_step); here every lane runs through the factors of its
+// channel side by side, picking each one's gate value with masks (and 1 past its last), so
+// there are no loops or branches that differ between lanes. The quad's currents are added in
+// channel order; absent channels are zeros.
+struct QuadChannels {
+    static constexpr int F = 4;      // factors with masks of their own; more run in a loop
+    DGate G;
+    const DGate *table;              // the gate table
+    int gate;                        // this lane's gate in it
+    bool mine;                       // this lane has a gate variable
+    float g, e, A;                   // channel s: Gbase, Erev (0 when absent), the compartment's area
+    uint32_t pick[F][NQ], one[F];    // factor m: all ones at its gate, or the bits of 1.0f
+    uint32_t powers;                 // the channel's power of gate j in byte j
+    int fmax;                        // most factors of a channel, over the wave's lanes
+
+    __device__ __forceinline__ void load(const DGate *__restrict__ gates, const CompConst &k, int qs) {
+        const int nq = (k.gmeta >> 24) & 7, nch = (k.gmeta >> 28) & 7;
+        mine = qs < nq;
+        table = gates;
+        A = k.A;
+        g = 0.0f;
+        e = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NCH; c++)
+            if (c == qs && c < nch) {
+                g = k.g[c];
+                e = k.e[c];
+            }
+        powers = 0;
+        int f = 0;
+#pragma unroll
+        for (int m = 0; m < F; m++) {
+            one[m] = 0x3F800000u;
+#pragma unroll
+            for (int j = 0; j < NQ; j++) pick[m][j] = 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < NQ; j++) {
+            const int cs = (k.gmeta >> (4 * j)) & 3, gi = (k.gmeta >> (4 * j + 2)) & 3;
+            const int at = (j < nq ? (k.chmeta >> (8 * cs)) & 0xFF : 0) * GATES_PER_TYPE + gi;
+            const DGate &Gj = gates[at];
+            if (j == qs) {
+                G = Gj;
+                gate = at;
+            }
+            const int inst = j < nq && cs == qs ? (Gj.forms >> 16) & 0xFF : 0;
+            powers |= (uint32_t)inst << (8 * j);
+#pragma unroll
+            for (int m = 0; m < F; m++)
+                if (m >= f && m < f + inst) {
+                    pick[m][j] = 0xFFFFFFFFu;
+                    one[m] = 0u;
+                }
+            f += inst;
+        }
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) f = max(f, __shfl_xor(f, m));
+        fmax = __builtin_amdgcn_readfirstlane(f);
+    }
+
+    __device__ __forceinline__ void currents(float qv, float V, float &I_ch, float &G_ch) const {
+        const float q[NQ] = {quad_bcast<0>(qv), quad_bcast<1>(qv), quad_bcast<2>(qv), quad_bcast<3>(qv)};
+        float f = 1.0f;      // conductance_scaling
+        if (fmax <= F) {
+            float x[F];
+#pragma unroll
+            for (int m = 0; m < F; m++) {
+                uint32_t b = one[m];
+#pragma unroll
+                for (int j = 0; j < NQ; j++) b |= __float_as_uint(q[j]) & pick[m][j];
+                x[m] = __uint_as_float(b);
+            }
+#pragma unroll
+            for (int m = 0; m < F; m++) f = f * x[m];
+        } else {
+            for (int j = 0; j < NQ; j++) {
+                const float qj = j == 0 ? q[0] : j == 1 ? q[1] : j == 2 ? q[2] : q[3];
+                for (int i = (powers >> (8 * j)) & 0xFF; i > 0; i--) f = f * qj;
+            }
+        }
+        const float Gscaled = g * f;
+        const float iDensity = Gscaled * (e - V) * 1e-5f;
+        const float gDensity = (Gscaled) * 1e-5f;
+        I_ch = 0.0f;
+        G_ch = 0.0f;
+        quad_add2(I_ch, G_ch, iDensity * A, gDensity * A);
+    }
+
+    // this lane's gate variable for the next step
+    __device__ __forceinline__ float next(float qv, float V, bool init, float dt) const {
+        // (the address formed where it is used)
+        int at = gate;
+        asm volatile("" : "+v"(at));
+        return mine ? gate_next(G, table + at, V, qv, init, dt) : qv;
+    }
+};
 
 __device__ __forceinline__ float pulses_current(const DevTables &T, const CompConst &k, int64_t gidx, float t) {
     // one pulse: 0 + (0 + amplitude) + 0 = amplitude exactly, or 0

@@ -1611,7 +1611,7 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 if (pf && first) HIPCHECK(ctx, hipEventRecord(ctx->pp0, ctx->stream));
                 if (ctx->point_quad) {
                     const int grid = (int)(((int64_t)ctx->n_point * 4 + tpb - 1) / tpb);
-                    void *args[] = {&T, &ctx->d_gates, &ctx->n_gates, &ctx->d_point, &n, (void *)&aa, (void *)&bb, &row0, &dt};
+                    void *args[] = {&T, &ctx->d_gates, &ctx->d_point, &n, (void *)&aa, (void *)&bb, &row0, &dt};
                     HIPCHECK(ctx, hipLaunchKernel(point_quad_kernel_ptr(), dim3(grid), dim3(tpb), args, 0, ctx->stream));
                 } else {
                     const int grid = (ctx->n_point + tpb - 1) / tpb;
