@@ -170,6 +170,13 @@ struct edenhip_ctx {
     unsigned long long *d_deliv_save = nullptr;
     int32_t *h_conflict = nullptr;   // pinned host copy of the conflict flag
     int64_t net_windows = 0, net_redone = 0;
+    bool net_quad = false;           // four lanes per cell (net_quad_kernel)
+    int net_groups = 0;              // groups of synapses it is built for (NET_QUAD_GROUPS)
+    NetClasses net_cls{};
+    NetRare *d_net_rare = nullptr;
+    bool net_free = false;           // no window can differ from step order: run without checks
+    int net_par = 0;                 // which of the two spike counters the next window uses
+    uint32_t *d_spk_count = nullptr;
     std::string kernel_name;
     std::vector<void *> allocs;
     // generic LEMS synapses: the run-time compiled synapse kernel and its tables
@@ -267,7 +274,8 @@ static std::vector<double> row_times(float dt, double t_final) {
     return ts;
 }
 
-static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std::vector<int32_t> &point);
+static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std::vector<int32_t> &point,
+                        const std::vector<DSynType> &stypes);
 
 // Scratch of edenhip_run_static: the tree kernels' work-queue counters (next task, finished
 // workgroups) of up to STATIC_QUEUE_BUCKETS buckets, in a file-scope device array that each
@@ -1308,14 +1316,15 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         HIPCHECK(ctx, hipEventCreate(&ctx->nw1));
     }
     HIPCHECK(ctx, hipEventCreateWithFlags(&ctx->ev_start, hipEventDisableTiming));
-    TRY(build_netwin(ctx, d, point));
+    TRY(build_netwin(ctx, d, point, st));
     HIPCHECK(ctx, hipDeviceSynchronize());
     return 0;
 }
 
 // Windowed network path: eligibility, per-compartment type runs, spike-target ring
 // addresses, second state copies. Models it does not cover keep the per-step path.
-static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std::vector<int32_t> &point) {
+static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std::vector<int32_t> &point,
+                        const std::vector<DSynType> &stypes) {
     if (!ctx->network || !ctx->buckets.empty() || ctx->opt.network_window == -1 || ctx->lems_fn || ctx->n_xcomp > 0)
         return 0;
     const int64_t NC = d->n_comps;
@@ -1390,7 +1399,7 @@ static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std
     TRY(alloc_zero(ctx, &N.poi_B[1], (size_t)n_poi));
     TRY(alloc_zero(ctx, &N.spike_mask, (size_t)NC));
     TRY(alloc_zero(ctx, &N.spk_list, (size_t)NC));
-    TRY(alloc_zero(ctx, &N.spk_count, 1));
+    TRY(alloc_zero(ctx, &ctx->d_spk_count, 2));
     TRY(alloc_zero(ctx, &N.conflict, 1));
     TRY(alloc_zero(ctx, &N.n_deliv, 1));
     TRY(alloc_zero(ctx, &ctx->d_deliv_save, 1));
@@ -1405,6 +1414,66 @@ static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std
         ctx->allocs.push_back(p);
         HIPCHECK(ctx, hipMemset(p, 0, bytes));
         ctx->snaps.push_back({N.ring, p, bytes});
+    }
+    // four lanes per cell: at most NET_CLASSES synapse types in all, of moderate parameters (its
+    // divisions and absent synapses' terms), NET_QUAD_MAX groups a wave and four Poisson inputs
+    // a cell; other networks take one lane per cell
+    {
+        NetClasses &K = ctx->net_cls;
+        std::vector<char> used(64, 0);
+        bool ok = true;
+        for (int64_t sq = 0; sq < d->comp_syn_begin[NC]; sq++) used[(size_t)d->syn_type[sq]] = 1;
+        for (int64_t pq = 0; pq < d->comp_poisson_begin[NC]; pq++) used[(size_t)d->poisson_syn_type[pq]] = 1;
+        for (int t = 0; t < d->n_syn_types && ok; t++) {
+            if (!used[(size_t)t]) continue;
+            const DSynType &st = stypes[(size_t)t];
+            const float jump = st.weight_prop * st.wf;
+            for (float x : {st.gbase, st.erev, jump}) ok = ok && std::fabs(x) < 0x1p60f;
+            for (float x : {st.tau_rise, st.tau_decay}) ok = ok && x > 0x1p-20f && x < 0x1p40f;
+            if (K.n == NET_CLASSES) { ok = false; break; }
+            const int c = K.n++;
+            auto recip = [](float x, double &hi, double &lo) {   // recip2
+                hi = 1.0 / (double)x;
+                lo = std::fma(-hi, (double)x, 1.0) / (double)x;
+            };
+            K.c[c] = NetClass{st.gbase, st.erev, jump, t, 0, 0, 0, 0};
+            recip(st.tau_rise, K.c[c].rise_hi, K.c[c].rise_lo);
+            recip(st.tau_decay, K.c[c].decay_hi, K.c[c].decay_lo);
+        }
+        int groups = 0;
+        for (size_t b0 = 0; b0 < point.size() && ok; b0 += 16) {
+            int32_t w[NET_CLASSES] = {};
+            for (size_t p = b0; p < std::min(point.size(), b0 + 16); p++) {
+                const int64_t g = point[p];
+                ok = ok && d->comp_poisson_begin[g + 1] - d->comp_poisson_begin[g] <= 4;
+                int32_t b = 0;
+                for (int r = 0; r < 4 && runs[g * 4 + r] != 0u; r++) {
+                    const int32_t e = (int32_t)(runs[g * 4 + r] & 0xFFFFu);
+                    for (int c = 0; c < K.n; c++)
+                        if (K.c[c].type == (int32_t)(runs[g * 4 + r] >> 16)) w[c] = std::max(w[c], (e - b + 15) / 16);
+                    b = e;
+                }
+            }
+            int tot = 0;
+            for (int32_t x : w) tot += x;
+            groups = std::max(groups, tot);
+        }
+        ctx->net_quad = ok && groups <= NET_QUAD_MAX;
+        for (int n : NET_QUAD_GROUPS)
+            if (ctx->net_groups < groups || ctx->net_groups == 0) ctx->net_groups = n;
+    }
+    if (ctx->net_quad) TRY(upload(ctx, &ctx->d_net_rare, std::vector<NetRare>(1, NetRare{ctx->T})));
+    // The one case a window cannot decide, a pending arrival that lies in two consecutive step
+    // windows [t, t + dt), needs windows that overlap. Where the float times do not, as with any
+    // dt of whole microseconds, no window has to be checked against step order.
+    {
+        const std::vector<double> ts = row_times(d->dt, d->t_final);
+        bool overlap = false;
+        for (size_t j = 0; j < ts.size() && !overlap; j++) {
+            const double next = j + 1 < ts.size() ? ts[j + 1] : ts[j] + (double)d->dt;
+            overlap = (float)ts[j] + d->dt > (float)next;
+        }
+        ctx->net_free = !overlap && ctx->opt.network_window != -2;
     }
     ctx->net_W = W;
     ctx->net_cur = 0;
@@ -1433,23 +1502,33 @@ static int net_copy_state(edenhip_ctx *ctx, int from, int to) {
 
 // One window [a, b) of the network path from state copy ctx->net_cur; with check, the
 // deliver pass first only checks that the window matches step-by-step order. Returns 1 in
-// *conflict when it does not (nothing committed then).
+// *conflict when it does not (nothing committed then). Without, the window kernel may clear the
+// ring words it consumes (no window is run again), which the deliver pass does otherwise.
 static int net_window(edenhip_ctx *ctx, int64_t a, int64_t b, int64_t row0, bool check, bool force, int *conflict,
                       int64_t *nl) {
-    NetTables &N = ctx->N;
+    NetTables N = ctx->N;
     DevTables T = ctx->T;
     const hipStream_t st = ctx->stream;
     float dt = ctx->dt;
     int cur = ctx->net_cur;
     int64_t last = ctx->total_rows;
-    HIPCHECK(ctx, hipMemsetAsync(N.spk_count, 0, sizeof(uint32_t), st));
+    // two spike counters take turns: a committing deliver pass zeroes the next window's
+    N.spk_count = ctx->d_spk_count + ctx->net_par;
+    N.spk_count_next = ctx->d_spk_count + (ctx->net_par ^ 1);
     int32_t np = ctx->n_point;
-    void *wargs[] = {&T, &N, &ctx->d_gates, &ctx->n_gates, &ctx->d_stypes, &ctx->n_stypes, &ctx->d_point, &np,
-                     &a, &b, &row0, &dt, &cur};
+    int clear = ctx->net_quad && !check ? 1 : 0;
     const bool prof = ctx->opt.profile != 0;
     if (prof) HIPCHECK(ctx, hipEventRecord(ctx->nw0, st));
-    HIPCHECK(ctx, hipLaunchKernel(net_window_kernel_ptr(), dim3(N.n_blocks), dim3(64), wargs,
-                                  (size_t)std::max(1, ctx->n_gates) * sizeof(DGate), st));
+    if (ctx->net_quad) {
+        void *wargs[] = {&T, &N, &ctx->d_gates, &ctx->net_cls, &ctx->d_net_rare, &ctx->d_point, &np, &a, &b, &row0, &dt,
+                         &cur, &clear};
+        HIPCHECK(ctx, hipLaunchKernel(net_quad_kernel_ptr(ctx->net_groups), dim3((np + 15) / 16), dim3(64), wargs, 0, st));
+    } else {
+        void *wargs[] = {&T, &N, &ctx->d_gates, &ctx->n_gates, &ctx->d_stypes, &ctx->n_stypes, &ctx->d_point, &np,
+                         &a, &b, &row0, &dt, &cur};
+        HIPCHECK(ctx, hipLaunchKernel(net_window_kernel_ptr(), dim3(N.n_blocks), dim3(64), wargs,
+                                      (size_t)std::max(1, ctx->n_gates) * sizeof(DGate), st));
+    }
     if (prof) {
         // the window kernel's own time (the delivery kernels are not included)
         HIPCHECK(ctx, hipEventRecord(ctx->nw1, st));
@@ -1460,32 +1539,49 @@ static int net_window(edenhip_ctx *ctx, int64_t a, int64_t b, int64_t row0, bool
         ctx->point_launches++;
     }
     (*nl)++;
-    const int grid = 1024;
-    int commit = 0;
+    // a workgroup per eight cells: a window of about a millisecond has fewer spiking cells, and
+    // the clearing of the ring needs the rest of the chip only in a large network
+    const int grid = std::min(1024, std::max(64, (np + 7) / 8));
+    int flags = 0;
     *conflict = 0;
     if (check) {
         HIPCHECK(ctx, hipMemsetAsync(N.conflict, 0, sizeof(int32_t), st));
-        void *dargs[] = {&T, &N, &a, &b, &last, &dt, &commit};
+        void *dargs[] = {&T, &N, &a, &b, &last, &dt, &flags};
         HIPCHECK(ctx, hipLaunchKernel(net_deliver_kernel_ptr(), dim3(grid), dim3(64), dargs, 0, st));
         HIPCHECK(ctx, hipMemcpyAsync(ctx->h_conflict, N.conflict, sizeof(int32_t), hipMemcpyDeviceToHost, st));
         HIPCHECK(ctx, hipStreamSynchronize(st));
         if (*ctx->h_conflict || force) {
+            HIPCHECK(ctx, hipMemsetAsync(N.spk_count, 0, sizeof(uint32_t), st));
             *conflict = 1;
             return 0;
         }
     }
-    commit = 1;
-    void *dargs[] = {&T, &N, &a, &b, &last, &dt, &commit};
+    flags = 1 | (clear ? 2 : 0);
+    void *dargs[] = {&T, &N, &a, &b, &last, &dt, &flags};
     HIPCHECK(ctx, hipLaunchKernel(net_deliver_kernel_ptr(), dim3(grid), dim3(64), dargs, 0, st));
     ctx->net_cur ^= 1;
+    ctx->net_par ^= 1;
     return 0;
 }
 
-// Steps [s0, s1) of a network through windows of up to net_W steps, each checked against
-// step-by-step order and, where it differs, run again one step at a time.
+// Steps [s0, s1) of a network through windows of up to net_W steps; where a window can differ
+// from step-by-step order (!net_free) each is checked and, if it does, run again one step at a
+// time.
 static int net_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0, int64_t *nl) {
     const hipStream_t st = ctx->stream;
-    for (int64_t a = s0; a < s1;) {
+    if (ctx->net_free) {
+        // an even number of windows of near-equal length leaves the state in copy 0
+        int64_t nw = (s1 - s0 + ctx->net_W - 1) / ctx->net_W;
+        if ((nw & 1) != ctx->net_cur && s1 - s0 > nw) nw++;
+        for (int64_t w = 0, a = s0; w < nw; w++) {
+            const int64_t b = a + (s1 - a) / (nw - w);
+            int conflict = 0;
+            TRY(net_window(ctx, a, b, row0, false, false, &conflict, nl));
+            ctx->net_windows++;
+            a = b;
+        }
+    }
+    for (int64_t a = ctx->net_free ? s1 : s0; a < s1;) {
         const int64_t b = std::min<int64_t>(s1, a + ctx->net_W);
         // event-log counters, restored if the window is run again
         HIPCHECK(ctx, hipMemcpyAsync(ctx->d_ev_save, ctx->T.n_events, sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
@@ -1991,9 +2087,9 @@ int edenhip_get_kernel_info(const edenhip_ctx *ctx, int32_t i, edenhip_kernel_in
     if (!ctx || !out || i < 0 || i >= edenhip_kernel_count(ctx)) return EDENHIP_E_INVALID;
     std::memset(out, 0, sizeof(*out));
     if (ctx->n_point > 0 && i == 0) {
-        std::snprintf(out->name, sizeof(out->name), ctx->netwin ? "net_window_kernel" : ctx->point_quad ? "point_quad_kernel" : "point_kernel");
+        std::snprintf(out->name, sizeof(out->name), ctx->netwin ? (ctx->net_quad ? "net_quad_kernel" : "net_window_kernel") : ctx->point_quad ? "point_quad_kernel" : "point_kernel");
         out->threads_per_block = 64;
-        out->grid = ctx->point_quad ? (int32_t)(((int64_t)ctx->n_point * 4 + 63) / 64) : (ctx->n_point + 63) / 64;
+        out->grid = ctx->point_quad || ctx->net_quad ? (int32_t)(((int64_t)ctx->n_point * 4 + 63) / 64) : (ctx->n_point + 63) / 64;
         out->n_cells = ctx->n_point;
         out->n_comps = ctx->n_point;
         out->launches = ctx->point_launches;

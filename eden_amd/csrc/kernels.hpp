@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "device_model.hpp"
+
 namespace edenhip {
 
 // One multi-compartment cell as seen by tree_kernel.
@@ -95,16 +97,42 @@ struct NetTables {
     float *poi_tsince[2], *poi_isi[2], *poi_A[2], *poi_B[2];
     uint64_t *spike_mask;          // [NC] spikes of the window, bit = step - window start
     int32_t *spk_list;             // compartments that spiked in the window
-    uint32_t *spk_count;
+    uint32_t *spk_count;           // this window's count; the deliver kernel zeroes the next one's
+    uint32_t *spk_count_next;
     const uint32_t *tgt_rw;        // per spike target (CSR spk_begin): ring word offset << 5 | bit
     int32_t *conflict;             // set when a window's result differs from step-by-step order
     unsigned long long *n_deliv;   // synaptic events received (spike-triggered), counted
 };
 
+// Device copy of the tables for what net_quad_kernel's step loop does seldom (events, Poisson
+// intervals, second pulses): read through a pointer there, so that the loop does not keep all
+// tables' addresses in registers.
+struct NetRare {
+    DevTables T;
+};
+
+// The synapse types a network uses, ascending, with what net_quad_kernel needs of each.
+constexpr int NET_CLASSES = 4;
+struct alignas(16) NetClass {
+    float gbase, erev, jump;       // jump: weight property * waveform factor
+    int32_t type;
+    double rise_hi, rise_lo, decay_hi, decay_lo;   // recip2 of the time constants
+};
+struct NetClasses {
+    int32_t n;                     // types in use, at most NET_CLASSES
+    NetClass c[NET_CLASSES];
+};
+
+// net_quad_kernel holds a wave's synapses in groups of four slots a lane (16 synapses a cell); it
+// is built for up to each of these numbers of groups. Registers: 8 a group.
+constexpr int NET_QUAD_GROUPS[] = {1, 2, 4, 6, 8, 10, 12, 16};
+constexpr int NET_QUAD_MAX = 16;
+
 // net: the variant for networks (synapses on tree compartments, spikes sent to recipients),
 // launched one step at a time; only without a channel wave.
 const void *tree_kernel_ptr(int tpb, bool split, bool net = false);
 const void *net_window_kernel_ptr();
+const void *net_quad_kernel_ptr(int groups);
 const void *net_deliver_kernel_ptr();
 const void *point_kernel_ptr();
 const void *ext_channels_kernel_ptr();
