@@ -152,6 +152,13 @@ struct edenhip_ctx {
     // initial copies of the state tables (for edenhip_reset)
     struct Snap { void *dst; void *src; size_t bytes; };
     std::vector<Snap> snaps;
+    Snap *d_snaps = nullptr;
+    int64_t snap_max = 0;                   // bytes of the largest
+    // reading back: the trace's rows in descriptor column order pass through d_rows in pieces
+    int32_t *d_desc_col = nullptr;
+    float *d_rows = nullptr;
+    int64_t rows_piece = 0;                 // rows that d_rows holds
+    bool ev_single = true;                  // each compartment has at most one event column
     // profiling
     double kernel_ms = 0;
     int64_t launches = 0;
@@ -321,6 +328,40 @@ __global__ void record_gates_kernel(DevTables T, const float *__restrict__ gq, c
     if (i >= n) return;
     const int64_t k = src[i] & REC_INDEX, kind = src[i] >> 60;
     trace_at(T, col[i], row) = kind == 0 ? T.q[k] : kind == 1 ? gq[k] : kind == 2 ? cs[k] : xq[k];
+}
+
+// Rows [r0, r0 + n) of the column-major trace as rows of descriptor columns, through 64 x 64
+// tiles in LDS: both sides move whole cache lines. (The host's transposition of a 16 MB trace
+// took 4 ms and its copies 2 ms; this takes 10 us and one copy.)
+__global__ void __launch_bounds__(256)
+trace_rows_kernel(const float *__restrict__ trace, int64_t stride, const int32_t *__restrict__ col, int64_t n_col,
+                  int64_t r0, int64_t n, float *__restrict__ out) {
+    __shared__ float tile[64][65];
+    const int64_t rb = (int64_t)blockIdx.x * 64, cb = (int64_t)blockIdx.y * 64;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int c = w; c < 64; c += 4)
+        if (cb + c < n_col && rb + lane < n) tile[c][lane] = trace[(int64_t)col[cb + c] * stride + r0 + rb + lane];
+    __syncthreads();
+    for (int r = w; r < 64; r += 4)
+        if (rb + r < n && cb + lane < n_col) out[(rb + r) * n_col + cb + lane] = tile[lane][r];
+}
+
+// Every state table back to its initial copy, and the output counters to zero: one launch in
+// place of a copy per table (a rewind of a small model 62 -> 3 us of the caller, 8 in all).
+__global__ void __launch_bounds__(256)
+restore_kernel(const edenhip_ctx::Snap *__restrict__ snaps, uint32_t *n_events, uint32_t *n_syn_events,
+               unsigned long long *n_deliv) {
+    const edenhip_ctx::Snap sn = snaps[blockIdx.y];
+    const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+    const int64_t n16 = (int64_t)sn.bytes / 16, n4 = (int64_t)sn.bytes / 4;
+    for (int64_t i = at; i < n16; i += step) static_cast<uint4 *>(sn.dst)[i] = static_cast<const uint4 *>(sn.src)[i];
+    for (int64_t i = 4 * n16 + at; i < n4; i += step)
+        static_cast<uint32_t *>(sn.dst)[i] = static_cast<const uint32_t *>(sn.src)[i];
+    if (blockIdx.y == 0 && at == 0) {
+        *n_events = 0u;
+        *n_syn_events = 0u;
+        if (n_deliv) *n_deliv = 0ull;
+    }
 }
 
 // Streams come from a per-device pool created once per process and kept until it ends:
@@ -1317,6 +1358,16 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     }
     HIPCHECK(ctx, hipEventCreateWithFlags(&ctx->ev_start, hipEventDisableTiming));
     TRY(build_netwin(ctx, d, point, st));
+    TRY(upload(ctx, &ctx->d_snaps, ctx->snaps));
+    for (const auto &sn : ctx->snaps) ctx->snap_max = std::max(ctx->snap_max, (int64_t)sn.bytes);
+    if (!ctx->desc_to_dev_col.empty()) {
+        // pieces of at most 16 MiB (one row where a row is longer)
+        const int64_t row = (int64_t)ctx->desc_to_dev_col.size() * 4;
+        ctx->rows_piece = std::max<int64_t>(1, std::min(ctx->chunk_rows, ((int64_t)16 << 20) / row));
+        TRY(upload(ctx, &ctx->d_desc_col, ctx->desc_to_dev_col));
+        TRY(alloc_zero(ctx, &ctx->d_rows, (size_t)(ctx->rows_piece * row / 4)));
+    }
+    for (const auto &e : ctx->ev_expand) ctx->ev_single = ctx->ev_single && e.size() <= 1;
     HIPCHECK(ctx, hipDeviceSynchronize());
     return 0;
 }
@@ -1898,11 +1949,12 @@ int edenhip_reset(edenhip_ctx *ctx) {
     if (!ctx) return EDENHIP_E_INVALID;
     if (!ctx->stream) return fail(ctx, EDENHIP_E_STATE, "context was not created successfully");
     HIPCHECK(ctx, hipSetDevice(ctx->device));
-    for (auto &s : ctx->snaps) HIPCHECK(ctx, hipMemcpyAsync(s.dst, s.src, s.bytes, hipMemcpyDeviceToDevice, ctx->stream));
-    HIPCHECK(ctx, hipMemsetAsync(ctx->T.n_events, 0, sizeof(uint32_t), ctx->stream));
-    HIPCHECK(ctx, hipMemsetAsync(ctx->T.n_syn_events, 0, sizeof(uint32_t), ctx->stream));
-    if (ctx->netwin) HIPCHECK(ctx, hipMemsetAsync(ctx->N.n_deliv, 0, sizeof(unsigned long long), ctx->stream));
-    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+    // (not waited for: later work follows on the same stream, and what reads on the host waits)
+    const unsigned blocks = (unsigned)std::min<int64_t>(2048, std::max<int64_t>(1, ctx->snap_max / (256 * 16 * 4)));
+    hipLaunchKernelGGL(restore_kernel, dim3(blocks, (unsigned)ctx->snaps.size()), dim3(256), 0, ctx->stream,
+                       (const edenhip_ctx::Snap *)ctx->d_snaps, ctx->T.n_events, ctx->T.n_syn_events,
+                       ctx->netwin ? ctx->N.n_deliv : nullptr);
+    HIPCHECK(ctx, hipGetLastError());
     ctx->rows_done = 0;
     ctx->next_step = -3;
     ctx->last_rows = 0;
@@ -1945,6 +1997,7 @@ int edenhip_get_state(edenhip_ctx *ctx, void *dst, int64_t bytes) {
     if (!ctx->stream) return fail(ctx, EDENHIP_E_STATE, "context was not created successfully");
     if (bytes < state_bytes(ctx)) return fail(ctx, EDENHIP_E_INVALID, "state buffer smaller than edenhip_state_size");
     HIPCHECK(ctx, hipSetDevice(ctx->device));
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
     char *p = static_cast<char *>(dst);
     StateHeader h{STATE_MAGIC, (int64_t)ctx->snaps.size(), state_bytes(ctx), ctx->next_step, ctx->rows_done};
     std::memcpy(p, &h, sizeof(h));
@@ -1978,6 +2031,7 @@ int edenhip_set_state(edenhip_ctx *ctx, const void *src, int64_t bytes) {
         p += 8 + sn.bytes;
     }
     HIPCHECK(ctx, hipSetDevice(ctx->device));
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
     p = static_cast<const char *>(src) + sizeof(h);
     for (const auto &sn : ctx->snaps) {
         p += 8;
@@ -1999,19 +2053,23 @@ int edenhip_read_trace(edenhip_ctx *ctx, float *dst, int64_t max_rows, int64_t *
     if (rows) *rows = nr;
     if (row0) *row0 = ctx->last_row0;
     if (nr <= 0 || ncol == 0 || !dst) return 0;
-    // device layout [column][chunk row]; the first nr rows of each column
-    const int64_t stride = ctx->chunk_rows;
-    std::vector<float> buf((size_t)(stride * ctx->n_dev_cols));
-    HIPCHECK(ctx, hipMemcpy(buf.data(), ctx->T.trace, buf.size() * sizeof(float), hipMemcpyDeviceToHost));
-    for (int64_t c = 0; c < ncol; c++) {
-        const float *src = buf.data() + (size_t)(ctx->desc_to_dev_col[c] * stride);
-        for (int64_t r = 0; r < nr; r++) dst[r * ncol + c] = src[r];
+    HIPCHECK(ctx, hipSetDevice(ctx->device));
+    for (int64_t r = 0; r < nr; r += ctx->rows_piece) {
+        const int64_t n = std::min(ctx->rows_piece, nr - r);
+        hipLaunchKernelGGL(trace_rows_kernel, dim3((unsigned)((n + 63) / 64), (unsigned)((ncol + 63) / 64)), dim3(256), 0,
+                           ctx->stream, (const float *)ctx->T.trace, ctx->chunk_rows, (const int32_t *)ctx->d_desc_col,
+                           ncol, r, n, ctx->d_rows);
+        HIPCHECK(ctx, hipGetLastError());
+        HIPCHECK(ctx, hipMemcpyAsync(dst + r * ncol, ctx->d_rows, (size_t)(n * ncol) * sizeof(float),
+                                     hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));   // the next piece reuses d_rows
     }
     return 0;
 }
 
 int edenhip_trace_device_ptr(edenhip_ctx *ctx, const float **dptr) {
     if (!ctx || !dptr) return EDENHIP_E_INVALID;
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
     *dptr = ctx->T.trace;
     return 0;
 }
@@ -2019,11 +2077,37 @@ int edenhip_trace_device_ptr(edenhip_ctx *ctx, const float **dptr) {
 int edenhip_read_events(edenhip_ctx *ctx, int64_t *col, int64_t *row, int64_t max_events, int64_t *n) {
     if (!ctx) return EDENHIP_E_INVALID;
     uint32_t cnt = 0;
-    HIPCHECK(ctx, hipMemcpy(&cnt, ctx->T.n_events, sizeof(cnt), hipMemcpyDeviceToHost));
+    HIPCHECK(ctx, hipSetDevice(ctx->device));
+    HIPCHECK(ctx, hipMemcpyAsync(&cnt, ctx->T.n_events, sizeof(cnt), hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
     if (cnt > ctx->T.max_events) return fail(ctx, EDENHIP_E_LIMIT, "event buffer overflow");
+    if (ctx->ev_single && !(col && row)) {   // one descriptor column each: the count alone
+        if (n) *n = cnt;
+        return 0;
+    }
     std::vector<int64_t> ev(cnt);
-    if (cnt) HIPCHECK(ctx, hipMemcpy(ev.data(), ctx->T.events, cnt * sizeof(int64_t), hipMemcpyDeviceToHost));
-    std::sort(ev.begin(), ev.end());
+    if (cnt) {
+        HIPCHECK(ctx, hipMemcpyAsync(ev.data(), ctx->T.events, cnt * sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+    }
+    // by (row, column): counted into rows, then the few events of each row sorted (many events),
+    // or sorted outright (few)
+    if ((int64_t)cnt * 4 > ctx->total_rows) {
+        std::vector<uint32_t> at((size_t)ctx->total_rows + 2, 0u);
+        for (int64_t x : ev) at[(size_t)(x >> 24) + 1]++;
+        for (size_t r = 1; r < at.size(); r++) at[r] += at[r - 1];
+        std::vector<int64_t> by_row(cnt);
+        for (int64_t x : ev) by_row[at[(size_t)(x >> 24)]++] = x;
+        ev.swap(by_row);
+        for (size_t b = 0; b < ev.size();) {
+            size_t e = b + 1;
+            while (e < ev.size() && (ev[e] >> 24) == (ev[b] >> 24)) e++;
+            std::sort(ev.begin() + (int64_t)b, ev.begin() + (int64_t)e);
+            b = e;
+        }
+    } else {
+        std::sort(ev.begin(), ev.end());
+    }
     int64_t k = 0;
     for (int64_t x : ev) {
         const int64_t r = x >> 24, c = x & 0xFFFFFF;
@@ -2033,7 +2117,7 @@ int edenhip_read_events(edenhip_ctx *ctx, int64_t *col, int64_t *row, int64_t ma
         }
     }
     // columns that share a compartment interleave: restore ascending column order per row
-    if (col && row) {
+    if (col && row && !ctx->ev_single) {
         const int64_t m = std::min(k, max_events);
         std::vector<std::pair<int64_t, int64_t>> pr((size_t)m);
         for (int64_t i = 0; i < m; i++) pr[i] = {row[i], col[i]};
@@ -2047,6 +2131,7 @@ int edenhip_read_events(edenhip_ctx *ctx, int64_t *col, int64_t *row, int64_t ma
 int edenhip_read_synapse_events(edenhip_ctx *ctx, int64_t *syn, int64_t *step, int64_t max_events, int64_t *n) {
     if (!ctx) return EDENHIP_E_INVALID;
     uint32_t cnt = 0;
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
     HIPCHECK(ctx, hipMemcpy(&cnt, ctx->T.n_syn_events, sizeof(cnt), hipMemcpyDeviceToHost));
     if (ctx->T.log_syn && cnt > ctx->T.max_syn_events) return fail(ctx, EDENHIP_E_LIMIT, "synaptic event log overflow");
     std::vector<int64_t> ev(cnt);
@@ -2062,6 +2147,7 @@ int edenhip_read_synapse_events(edenhip_ctx *ctx, int64_t *syn, int64_t *step, i
 
 int edenhip_get_voltages(edenhip_ctx *ctx, float *dst) {
     if (!ctx || !dst) return EDENHIP_E_INVALID;
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
     HIPCHECK(ctx, hipMemcpy(dst, ctx->T.V, ctx->NC * sizeof(float), hipMemcpyDeviceToHost));
     return 0;
 }
@@ -2130,6 +2216,7 @@ int edenhip_network_stats(edenhip_ctx *ctx, int32_t *window_steps, int64_t *wind
     if (windows_rerun) *windows_rerun = ctx->net_redone;
     if (synaptic_events) {
         unsigned long long n = 0;
+        HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->netwin) HIPCHECK(ctx, hipMemcpy(&n, ctx->N.n_deliv, sizeof(n), hipMemcpyDeviceToHost));
         *synaptic_events = ctx->netwin ? (int64_t)n : -1;
     }

@@ -423,18 +423,17 @@ class Simulation:
 
     def run_all(self):
         """Run every row; return the full trace [rows x n_record]."""
-        parts = []
-        while True:
+        out = np.empty((self.total_rows, self.n_record), np.float32)
+        rows, row0, filled = C.c_int64(), C.c_int64(), 0
+        while filled < self.total_rows:
             n = self.run(-1)
             if n == 0:
                 break
-            tr, _ = self.read_trace()
-            parts.append(tr.copy())
-            if sum(p.shape[0] for p in parts) >= self.total_rows:
-                break
-        if not parts:
-            return np.zeros((0, self.n_record), np.float32)
-        return np.concatenate(parts, axis=0)
+            if self.n_record:
+                self._check(self.lib.edenhip_read_trace(self.h, C.c_void_p(out.ctypes.data + 4 * filled * self.n_record),
+                                                        n, C.byref(rows), C.byref(row0)), "read_trace")
+            filled += n
+        return out if filled == self.total_rows else out[:filled].copy()
 
     def read_events(self):
         n = C.c_int64()
