@@ -494,12 +494,13 @@ struct CompConst {
 };
 
 // A tree-cell compartment that is not simple: its constants and compartment word, staged
-// per cell (80 bytes, read with 16-byte loads).
+// per cell (96 bytes, read with 16-byte loads).
 struct alignas(16) TreeComplex {
     CompConst k;
     uint32_t tcm;
+    double rC;      // 1 / C (div_c)
 };
-static_assert(sizeof(TreeComplex) == 80, "TreeComplex layout");
+static_assert(sizeof(TreeComplex) == 96, "TreeComplex layout");
 
 __device__ __forceinline__ void load_comp_const(const DevTables &T, int64_t gidx, CompConst &k) {
     k.C = T.C[gidx]; k.A = T.A[gidx]; k.invrc = T.invrc[gidx]; k.vthr = T.vthr[gidx];

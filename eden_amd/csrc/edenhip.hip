@@ -882,6 +882,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
             }
             x.k.rec = rec_col[g]; x.k.ev = ev_col[g];
             x.tcm = tcm[g];
+            x.rC = 1.0 / (double)C[g];
             const int32_t idx = (int32_t)(cxv.size() - (size_t)tc.cx_off);
             if (idx > 0xFFFF) return fail(ctx, EDENHIP_E_LIMIT, "more than 65536 complex compartments in a cell");
             cflag[g] = TCX_COMPLEX | (uint32_t)idx;

@@ -230,6 +230,10 @@ __device__ __forceinline__ void channel_phase(const DGate *gates, const uint32_t
 // either in the cable group after the membrane phase, or, with SPLIT, in one extra wave at
 // the same time as the cable group's step; voltages and open fractions are then
 // double-buffered and the two meet at one workgroup barrier per step.
+// A step is bound by the latency of its rounds, one wave's dependent trips through LDS: a round
+// takes its header from a lane, reads everything before its first use and divides by constants
+// through double (div_c); the root's update runs its channels on a quad (QuadChannels). 7 trees of up
+// to 300 compartments, 1,004 steps and their rows read: 4.1 -> 3.6 ms.
 // NET: networks, launched one step at a time. A compartment with chemical synapses
 // (TCM_SYN) runs them in its complex update, with the trigger flags of the step's parity as
 // the point kernel does, and a compartment with spike recipients sends its spikes to the
@@ -298,64 +302,62 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
         // Hines task lists (tree_schedule.hpp, plan_tree_waves): cable wave wv runs the lists
         // of its subtrees, wave 0 also those of the junction. run_list calls body(word) round
         // after round with no barrier (a wave's LDS accesses are performed in order), on the
-        // lanes below the round's task count; lanes beyond it are masked off (their word is
-        // the idle word, which points every access at the dummy slot N). Task words hold byte
-        // offsets of node records, which start at a constant LDS address. Every lane reads a word
-        // from the round (the block ends with padding for the lanes beyond a round's count).
-        // The loop is unrolled twice, so that no register moves between rounds: after a
-        // round's body is issued, the words of the round after next and the header of the
-        // round two after that are read into the registers the round had used (five sentinel
-        // headers end the block). Each value is then complete before its use, with no wait on
-        // the loads just issued.
+        // lanes below the round's task count. Task words hold byte offsets of node records, which
+        // start at a constant LDS address. Every lane reads a word from the round (the block ends
+        // with padding for the lanes beyond a round's count).
+        // A list's round headers are kept a lane each (read again every 62 rounds), so a round
+        // takes its header from a lane instead of from LDS. The loop is unrolled twice: after a
+        // round's body is issued, the words of the round after next are read into the registers
+        // that the round had used, complete before their use and with no register moved.
         constexpr int W = TPB / 64;
         const int wv = tid >> 6, lane = tid & 63;
         const uint32_t dummy_off = 16u * (uint32_t)N;
-        const uint2 idle_fold = make_uint2(dummy_off | (dummy_off << 16), dummy_off);
-        const uint2 idle_bwd = make_uint2(dummy_off | (dummy_off << 16), dummy_off);
-        // constant trees take four-word fold tasks with merged children (plan_tree_waves
-        // with merge): c0, c1 and the grandchildren refolded through each, dummy where absent
-        const uint32_t dd = dummy_off | (dummy_off << 16);
-        const uint4 idle_fold4 = make_uint4(dd, dd, dd, dummy_off);
         char *const dxb = nodes;       // task words: byte offsets 16 p of node records
         char *const ub = nodes + 8;
-        // a list's directory entry and first four round headers: the same every step, so they
-        // are read once per cell into scalar registers, and a list starts with the reads of its
-        // first task words
-        struct ListHead {
-            uint32_t list, h0, h1, h2, h3;
+        struct List {
+            int first, cnt;     // first round header, rounds
+            uint32_t hv;        // lane r: header r
         };
-        auto list_head = [&](int dir) {
-            ListHead L;
-            L.list = __builtin_amdgcn_readfirstlane(sW[dir]);
-            const int first = L.list & 0xFFFFu;
-            L.h0 = __builtin_amdgcn_readfirstlane(sW[first]);
-            L.h1 = __builtin_amdgcn_readfirstlane(sW[first + 1]);
-            L.h2 = __builtin_amdgcn_readfirstlane(sW[first + 2]);
-            L.h3 = __builtin_amdgcn_readfirstlane(sW[first + 3]);
+        auto load_list = [&](int dir) {
+            List L;
+            const uint32_t e = __builtin_amdgcn_readfirstlane(sW[dir]);
+            L.first = e & 0xFFFFu;
+            L.cnt = e >> 16;
+            L.hv = sW[L.first + lane];
             return L;
         };
-        auto run_list = [&](const ListHead &L, auto idle, auto body) {
-            using Word = decltype(idle);
-            const int first = L.list & 0xFFFFu, cnt = L.list >> 16;
-            auto word = [&](uint32_t h, bool &act) {
-                const Word w = reinterpret_cast<const Word *>(sW + (h & 0xFFFFu))[lane];
-                act = lane < (int)(h >> 16);
-                return act ? w : idle;
-            };
-            bool aa, ab;
-            uint32_t ha = L.h2, hb = L.h3;
-            Word wa = word(L.h0, aa), wb = word(L.h1, ab);
-            for (int r = 0; r < cnt; r += 2) {
-                if (aa) body(wa);
-                wa = word(ha, aa);
-                ha = sW[first + r + 4];
-                if (r + 1 < cnt) {
-                    if (ab) body(wb);
-                    wb = word(hb, ab);
-                    hb = sW[first + r + 5];
+        auto run_list = [&](const List &L, auto type, auto body) {
+            using Word = decltype(type);
+            if (L.cnt == 0) return;
+            uint32_t hv = L.hv;
+            int hbase = 0;
+            auto head = [&](int r) -> uint32_t {
+                if (__builtin_expect(r - hbase >= 64, 0)) {
+                    // (read and used here, so that the usual way waits for no LDS access)
+                    hbase = r;
+                    hv = sW[L.first + r + lane];
+                    return (uint32_t)__builtin_amdgcn_readlane(hv, 0);
                 }
+                return (uint32_t)__builtin_amdgcn_readlane(hv, r - hbase);
+            };
+            auto word = [&](uint32_t h) { return reinterpret_cast<const Word *>(sW + (h & 0xFFFFu))[lane]; };
+            uint32_t ha = head(0), hb = head(1);
+            Word wa = word(ha), wb = word(hb);
+            for (int r = 0;;) {
+                if ((uint32_t)lane < (ha >> 16)) body(wa);
+                if (++r >= L.cnt) break;
+                ha = head(r + 1);
+                wa = word(ha);
+                if ((uint32_t)lane < (hb >> 16)) body(wb);
+                if (++r >= L.cnt) break;
+                hb = head(r + 1);
+                wb = word(hb);
             }
         };
+        // constant trees take four-word fold tasks with merged children (plan_tree_waves
+        // with merge): c0, c1 and the grandchildren refolded through each, dummy where absent
+        const uint4 fold4{};
+        const uint2 fold2{}, bwd2{};
         for (int i = tid; i < N; i += NT) sU(i) = u_g[c0 + i];
         for (int i = tid; i < NG; i += NT) {
             sQ[i] = gq_g[gq0 + i];
@@ -369,7 +371,7 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
         if (cxmax_lds > 0) {
             const uint4 *src = reinterpret_cast<const uint4 *>(cx_g + cell.cx_off);
             uint4 *dst = reinterpret_cast<uint4 *>(sCX);
-            for (int i = tid; i < cell.n_cx * 5; i += NT) dst[i] = src[i];
+            for (int i = tid; i < cell.n_cx * (int)(sizeof(TreeComplex) / 16); i += NT) dst[i] = src[i];
             CX = sCX;
         }
         // voltages read from LDS: the root's in a constant tree (no gated channel or input
@@ -388,17 +390,19 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
         // per-step operation order). A complex compartment's constants come from its record.
         // Slots beyond the cell behave as simple compartments with no channel conductance,
         // C = 1 and the dummy position N, so they compute exactly the dummy slot's (1, 0).
-        float V[K], g0[K], e0[K], Ar[K], Cr[K], Gs[K], Ds[K];
+        float V[K], g0[K], e0[K], Ar[K], Gs[K], Ds[K];
+        double rC[K];           // 1 / C (div_c)
         // fl: the compartment's flag word (TCX_COMPLEX | record index, or 0) | BFS position << 16
         uint32_t fl[K];
         auto posof = [&](int j) { return (int)((fl[j] >> 16) & 0x7FFu); };
-        bool slot_any[K], slot_simple[K];   // per wave and slot: any valid lane, no complex lane
+        bool slot_any[K], slot_simple[K], slot_cx[K];   // per wave and slot: any valid lane, no complex
+                                                        // lane but the root's, any complex lane
         const int wbase = __builtin_amdgcn_readfirstlane(tid & ~63);
 #pragma unroll
         for (int j = 0; j < K; j++) {
             const int c = tid + TPB * j;
             const bool valid = cable && c < N;
-            V[j] = 0.0f; g0[j] = 0.0f; e0[j] = 0.0f; Ar[j] = 0.0f; Cr[j] = 1.0f; Gs[j] = 0.0f; Ds[j] = 1.0f;
+            V[j] = 0.0f; g0[j] = 0.0f; e0[j] = 0.0f; Ar[j] = 0.0f; rC[j] = 1.0; Gs[j] = 0.0f; Ds[j] = 1.0f;
             fl[j] = (uint32_t)N << 16;
             if (valid) {
                 const int64_t g = c0 + c;
@@ -408,10 +412,10 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                     g0[j] = T.chg[g * NCH];
                     e0[j] = T.che[g * NCH];
                     Ar[j] = T.A[g];
-                    Cr[j] = T.C[g];
+                    rC[j] = 1.0 / (double)T.C[g];
                     const float G_ch = 0.0f + (((g0[j] * 1.0f) * 1e-5f) * Ar[j]);
                     const float G_int = (G_ch + 0.0f) + 0.0f;
-                    const float Dd = 1 * (G_int / Cr[j]) + T.invrc[g];
+                    const float Dd = 1 * (G_int / T.C[g]) + T.invrc[g];
                     Gs[j] = G_int;
                     Ds[j] = 1 + Dd * dt;
                 }
@@ -419,11 +423,13 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
             slot_any[j] = __builtin_amdgcn_readfirstlane(wbase + TPB * j) < N && cable;
             // the root (thread 0, slot 0) is updated separately, after wave 0's fold rounds
             slot_simple[j] = __ballot(valid && c != 0 && (fl[j] & TCX_COMPLEX)) == 0ull;
+            slot_cx[j] = __ballot(valid && (fl[j] & TCX_COMPLEX)) != 0ull;
         }
         __syncthreads();
         // the Hines lists of this wave (for the channel wave, unused) and of the junction
-        const ListHead Lf = list_head(2 * wv), Lb = list_head(2 * wv + 1);
-        const ListHead Ljf = list_head(2 * W), Ljb = list_head(2 * W + 1);
+        const int lw = cable ? wv : 0;
+        const List Lf = load_list(2 * lw), Lb = load_list(2 * lw + 1);
+        const List Ljf = load_list(2 * W), Ljb = load_list(2 * W + 1);
         if (const_tree) {
             // eliminated diagonals of the constant subtrees: the forward sweep's diagonal part
             // on this step-independent matrix, with the per-step operations
@@ -466,9 +472,9 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                 const float2 ubb = *reinterpret_cast<const float2 *>(ub + bo);
                 reinterpret_cast<float2 *>(dxb + po)->x = (d - (ua.y / da) * ua.x) - (ubb.y / db) * ubb.x;
             };
-            if (cable) run_list(Lf, idle_fold4, diag_task);
+            if (cable) run_list(Lf, fold4, diag_task);
             __syncthreads();
-            if (cable && wv == 0) run_list(Ljf, idle_fold4, diag_task);
+            if (cable && wv == 0) run_list(Ljf, fold4, diag_task);
             __syncthreads();
             // from here on, below the root: sDX[c] = (ratio Uj / D', right-hand side) and
             // sU[c] = (Ui, D'); the per-step diagonal register Ds holds the ratio
@@ -533,10 +539,45 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
             }
             const float I_int = I_ch + I_in + I_syn;
             const float G_int = G_ch + G_in + G_syn;
-            const float Dd = 1 * (G_int / k.C) + k.invrc;
+            const float Dd = 1 * div_c(G_int, cx.rC) + k.invrc;
             Dn = (const_tree && posof(j) != 0) ? Ds[j] : 1 + Dd * dt;
-            Vn = init ? V[j] : V[j] + (dt * (I_int + ((V[j] * G_int)))) / k.C;
+            Vn = init ? V[j] : V[j] + div_c(dt * (I_int + ((V[j] * G_int))), cx.rC);
         };
+        // The root's update runs on the first quad of wave 0, a channel a lane (channel c's density
+        // and its place in sF on lane c), the currents added in channel order by quad_add2, as on
+        // point cells. A root with inputs, synapses or channels from elsewhere keeps the general
+        // update on one lane, and so does a simple one (whose terms are constants).
+        bool root_quad = false;
+        float rk_g = 0.0f, rk_e = 0.0f, rk_A = 0.0f, rk_inv = 0.0f, rk_p0s = 0.0f, rk_p0e = -1.0f, rk_p0a = 0.0f;
+        int rk_f = -1;
+        double rk_rC = 1.0;
+        if (wv == 0 && cable) {
+            const uint32_t rf = __builtin_amdgcn_readfirstlane(fl[0]);
+            if (rf & TCX_COMPLEX) {
+                const TreeComplex &cx = CX[rf & 0xFFFFu];
+                root_quad = !(cx.tcm & (TCM_INPUT | TCM_SYN | TCM_XCH)) && !(cx.k.gmeta & GM_MORE_PULSES);
+                const int nch = cx.tcm & 7;
+                const uint32_t mask = (cx.tcm >> 3) & 15;
+                int idx = cx.tcm >> 16;
+#pragma unroll
+                for (int c = 0; c < NCH; c++) {
+                    const bool gated = (mask >> c) & 1;
+                    if (lane == c && c < nch) {
+                        rk_g = cx.k.g[c];
+                        rk_e = cx.k.e[c];
+                        rk_f = gated ? idx : -1;
+                    }
+                    idx += gated ? 1 : 0;
+                }
+                rk_A = cx.k.A;
+                rk_inv = cx.k.invrc;
+                rk_rC = cx.rC;
+                rk_p0s = cx.k.p0s;
+                rk_p0e = cx.k.p0e;
+                rk_p0a = cx.k.p0a;
+            }
+        }
+        root_quad = __builtin_amdgcn_readfirstlane(root_quad);
         int cur = 0, fcur = 0;
         if (SPLIT && !cable) {
             // channel wave, in a step loop of its own (so that none of the cable group's
@@ -606,7 +647,7 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                         const float I_ch_s = 0.0f + ((((g0[j] * 1.0f) * (e0[j] - V[j])) * 1e-5f) * Ar[j]);
                         const float I_int_s = (I_ch_s + 0.0f) + 0.0f;
                         float Dn = Ds[j];
-                        float Vn = init ? V[j] : V[j] + (dt * (I_int_s + ((V[j] * Gs[j])))) / Cr[j];
+                        float Vn = init ? V[j] : V[j] + div_c(dt * (I_int_s + ((V[j] * Gs[j]))), rC[j]);
                         if (!slot_simple[j] && c != 0 && (fl[j] & TCX_COMPLEX)) complex_update(j, c, sF, t, init, s, Dn, Vn);
                         sDX(posof(j)) = make_float2(Dn, Vn);
                     }
@@ -628,17 +669,16 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                         // reads the same values and writes that child in the same round
                         auto fold_const = [&](uint4 w) {
                             const uint32_t po = w.x & 0xFFFFu, ao = w.x >> 16, bo = w.y & 0xFFFFu;
-                            auto rhs = [&](float x, uint32_t g0, uint32_t g1) {
-                                const float2 q0 = *reinterpret_cast<const float2 *>(dxb + g0);
-                                const float2 q1 = *reinterpret_cast<const float2 *>(dxb + g1);
-                                return (x - q0.x * q0.y) - q1.x * q1.y;
-                            };
-                            const float2 a = *reinterpret_cast<const float2 *>(dxb + ao);
-                            const float2 b = *reinterpret_cast<const float2 *>(dxb + bo);
-                            const float xa = rhs(a.y, w.y >> 16, w.z & 0xFFFFu);
-                            const float xb = rhs(b.y, w.z >> 16, w.w);
+                            auto at = [&](uint32_t o) { return *reinterpret_cast<const float2 *>(dxb + o); };
+                            // (every read before the first use)
+                            const float2 a = at(ao), a0 = at(w.y >> 16), a1 = at(w.z & 0xFFFFu);
+                            const float2 b = at(bo), b0 = at(w.z >> 16), b1 = at(w.w);
                             float *xp = reinterpret_cast<float *>(dxb + po) + 1;
-                            *xp = (*xp - a.x * xa) - b.x * xb;
+                            const float x = *xp;
+                            __builtin_amdgcn_sched_barrier(0);
+                            const float xa = (a.y - a0.x * a0.y) - a1.x * a1.y;
+                            const float xb = (b.y - b0.x * b0.y) - b1.x * b1.y;
+                            *xp = (x - a.x * xa) - b.x * xb;
                         };
                         // general tree: diagonal and right-hand side
                         auto fold_task = [&](uint2 w) {
@@ -662,31 +702,37 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                         // first form, whose extra solve is discarded
                         auto bwd_task = [&](uint2 w) {
                             const uint32_t po = w.x & 0xFFFFu, so = w.x >> 16, mo = w.y;
+                            // node records: x ratio or diagonal, y rhs, z Ui, w D' (constant tree)
                             const float xs = reinterpret_cast<const float2 *>(dxb + so)->y;
-                            const float2 dm = *reinterpret_cast<const float2 *>(dxb + mo);
-                            const float2 um = *reinterpret_cast<const float2 *>(ub + mo);
-                            const float2 dp = *reinterpret_cast<const float2 *>(dxb + po);
-                            const float2 up = *reinterpret_cast<const float2 *>(ub + po);
-                            float xm, x;
-                            if (const_tree) {
-                                // sU[c] = (Ui, D')
-                                xm = (dm.y - um.x * xs) / um.y;
-                                xm = mo == dummy_off ? xs : xm;
-                                x = (dp.y - up.x * xm) / up.y;
-                            } else {
-                                xm = (dm.y - um.x * xs) / dm.x;
-                                xm = mo == dummy_off ? xs : xm;
-                                x = (dp.y - up.x * xm) / dp.x;
-                            }
-                            reinterpret_cast<float2 *>(dxb + po)->y = x;
+                            const float4 m = *reinterpret_cast<const float4 *>(dxb + mo);
+                            const float4 p = *reinterpret_cast<const float4 *>(dxb + po);
+                            __builtin_amdgcn_sched_barrier(0);
+                            float xm = (m.y - m.z * xs) / (const_tree ? m.w : m.x);
+                            xm = mo == dummy_off ? xs : xm;
+                            reinterpret_cast<float2 *>(dxb + po)->y = (p.y - p.z * xm) / (const_tree ? p.w : p.x);
                         };
                         if (const_tree)
-                            run_list(Lf, idle_fold4, fold_const);
+                            run_list(Lf, fold4, fold_const);
                         else
-                            run_list(Lf, idle_fold, fold_task);
-                        if (tid == 0 && (fl[0] & TCX_COMPLEX)) {
-                            // the root compartment's update, left out of the compartment phase: only
-                            // the root fold reads the root's diagonal and right-hand side
+                            run_list(Lf, fold2, fold_task);
+                        // the root compartment's update, left out of the compartment phase: only
+                        // the root fold reads the root's diagonal and right-hand side
+                        if (root_quad) {
+                            const float Vr = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(V[0])));
+                            const float f = rk_f >= 0 ? sF[rk_f] : 1.0f;
+                            const float Gscaled = rk_g * f;
+                            const float iDensity = Gscaled * (rk_e - Vr) * 1e-5f;
+                            const float gDensity = (Gscaled) * 1e-5f;
+                            float I_ch = 0.0f, G_ch = 0.0f;
+                            quad_add2(I_ch, G_ch, iDensity * rk_A, gDensity * rk_A);
+                            const float I_in = (rk_p0s <= t && t <= rk_p0e) ? rk_p0a : 0.0f, G_in = 0.0f;
+                            const float I_syn = 0.0f, G_syn = 0.0f;
+                            const float I_int = I_ch + I_in + I_syn;
+                            const float G_int = G_ch + G_in + G_syn;
+                            const float Dd = 1 * div_c(G_int, rk_rC) + rk_inv;
+                            const float Vn = Vr + div_c(dt * (I_int + ((Vr * G_int))), rk_rC);
+                            if (tid == 0) sDX(0) = make_float2(1 + Dd * dt, Vn);
+                        } else if (tid == 0 && (fl[0] & TCX_COMPLEX)) {
                             float Dn = Ds[0], Vn = V[0];
                             complex_update(0, 0, sF, t, false, s, Dn, Vn);
                             sDX(0) = make_float2(Dn, Vn);
@@ -699,21 +745,22 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                             // it would hold back, config 2 was slower)
                             if constexpr (!SPLIT) __builtin_amdgcn_s_setprio(3);
                             if (const_tree)
-                                run_list(Ljf, idle_fold4, fold_const);
+                                run_list(Ljf, fold4, fold_const);
                             else
-                                run_list(Ljf, idle_fold, fold_task);
+                                run_list(Ljf, fold2, fold_task);
                             if (lane == 0) {
                                 // the root: all its children (positions 1 .. nr) in order, loads
                                 // issued four at a time, then its solve
                                 const int nr = cell.root_children;
                                 float2 r0 = sDX(0);
-                                int c = 1;
-                                for (; c + 3 <= nr; c += 4) {
+                                for (int c = 1; c <= nr; c += 4) {
+                                    // (the dummy slot past the last child: its terms are zero)
                                     float2 a[4], u[4];
     #pragma unroll
                                     for (int k = 0; k < 4; k++) {
-                                        a[k] = sDX(c + k);
-                                        u[k] = sU(c + k);
+                                        const int p = c + k <= nr ? c + k : N;
+                                        a[k] = sDX(p);
+                                        u[k] = sU(p);
                                     }
     #pragma unroll
                                     for (int k = 0; k < 4; k++) {
@@ -722,42 +769,38 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                                         r0.y = r0.y - r * a[k].y;
                                     }
                                 }
-                                for (; c <= nr; c++) {
-                                    const float2 a = sDX(c), u = sU(c);
-                                    const float r = const_tree ? a.x : u.y / a.x;
-                                    r0.x = r0.x - r * u.x;
-                                    r0.y = r0.y - r * a.y;
-                                }
                                 r0.y = r0.y / r0.x;
                                 sDX(0) = r0;
                             }
-                            run_list(Ljb, idle_bwd, bwd_task);
+                            run_list(Ljb, bwd2, bwd_task);
                             if constexpr (!SPLIT) __builtin_amdgcn_s_setprio(0);
                         }
                         lds_barrier<TPB>();
-                        run_list(Lb, idle_bwd, bwd_task);
+                        run_list(Lb, bwd2, bwd_task);
                         lds_barrier<TPB>();
                     }
+                    // new voltages: every slot's read in flight (slots beyond the cell read the
+                    // dummy), then spikes and traces where the wave has complex compartments
+                    float Vn[K];
+    #pragma unroll
+                    for (int j = 0; j < K; j++) Vn[j] = init || !slot_any[j] ? V[j] : sDX(posof(j)).y;
     #pragma unroll
                     for (int j = 0; j < K; j++) {
                         const int c = tid + TPB * j;
-                        if (slot_any[j] && c < N) {
-                            const float Vn = init ? V[j] : sDX(posof(j)).y;
-                            if (fl[j] & TCX_COMPLEX) {
-                                const TreeComplex &cx = CX[fl[j] & 0xFFFFu];
-                                // a recorded compartment is complex: its trace column is in its
-                                // record; the trace row of step s holds the voltage the step
-                                // started from
-                                if (!init && cx.k.rec >= 0) trace_at(T, cx.k.rec, s - 1 - row0) = V[j];
-                                const float vthr = cx.k.vthr;
-                                if (V[j] < vthr && vthr < Vn) {
-                                    log_event(T, cx.k.ev, s);
-                                    if constexpr (NET) send_spike(T, c0 + c, (int)((s + 3) & 1) ^ 1);
-                                }
+                        if (slot_cx[j] && (fl[j] & TCX_COMPLEX)) {
+                            const TreeComplex &cx = CX[fl[j] & 0xFFFFu];
+                            // a recorded compartment is complex: its trace column is in its
+                            // record; the trace row of step s holds the voltage the step
+                            // started from
+                            if (!init && cx.k.rec >= 0) trace_at(T, cx.k.rec, s - 1 - row0) = V[j];
+                            const float vthr = cx.k.vthr;
+                            if (V[j] < vthr && vthr < Vn[j]) {
+                                log_event(T, cx.k.ev, s);
+                                if constexpr (NET) send_spike(T, c0 + c, (int)((s + 3) & 1) ^ 1);
                             }
-                            V[j] = Vn;
-                            if (c < NV) sVn[c] = Vn;
                         }
+                        V[j] = Vn[j];
+                        if (slot_any[j] && c < NV) sVn[c] = Vn[j];
                     }
                 }
                 // the next step reads voltages and open fractions written above by other lanes
@@ -789,52 +832,20 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
     }
 }
 
-#define EDENHIP_TREE_INST(TPB, SPLIT, NET)                                                                         \
-    template __global__ void tree_kernel<TPB, SPLIT, NET>(                                                         \
-        DevTables, const DGate *, int, const DSynType *, int, const TreeCell *, const int32_t *, int32_t, int32_t *,  \
-        const uint32_t *, const int32_t *, const float2 *, const uint32_t *, const uint32_t *, float *,             \
-        const uint32_t *, const uint32_t *, const uint32_t *, const TreeComplex *, int32_t, int32_t, int32_t, int32_t, \
-        int32_t, int32_t, int32_t, int64_t, int64_t, int64_t, float);
-EDENHIP_TREE_INST(64, true, false)
-EDENHIP_TREE_INST(64, false, false)
-EDENHIP_TREE_INST(128, true, false)
-EDENHIP_TREE_INST(128, false, false)
-EDENHIP_TREE_INST(256, true, false)
-EDENHIP_TREE_INST(256, false, false)
-EDENHIP_TREE_INST(512, true, false)
-EDENHIP_TREE_INST(512, false, false)
-EDENHIP_TREE_INST(64, false, true)
-EDENHIP_TREE_INST(128, false, true)
-EDENHIP_TREE_INST(256, false, true)
-EDENHIP_TREE_INST(512, false, true)
-
-const void *tree_kernel_ptr(int tpb, bool split, bool net) {
-    if (net) {
-        if (split) return nullptr;
-        switch (tpb) {
-        case 64: return reinterpret_cast<const void *>(&tree_kernel<64, false, true>);
-        case 128: return reinterpret_cast<const void *>(&tree_kernel<128, false, true>);
-        case 256: return reinterpret_cast<const void *>(&tree_kernel<256, false, true>);
-        case 512: return reinterpret_cast<const void *>(&tree_kernel<512, false, true>);
-        default: return nullptr;
-        }
-    }
-    if (split) {
-        switch (tpb) {
-        case 64: return reinterpret_cast<const void *>(&tree_kernel<64, true, false>);
-        case 128: return reinterpret_cast<const void *>(&tree_kernel<128, true, false>);
-        case 256: return reinterpret_cast<const void *>(&tree_kernel<256, true, false>);
-        case 512: return reinterpret_cast<const void *>(&tree_kernel<512, true, false>);
-        default: return nullptr;
-        }
-    }
+template <bool SPLIT, bool NET>
+static const void *tree_kernel_of(int tpb) {
     switch (tpb) {
-    case 64: return reinterpret_cast<const void *>(&tree_kernel<64, false, false>);
-    case 128: return reinterpret_cast<const void *>(&tree_kernel<128, false, false>);
-    case 256: return reinterpret_cast<const void *>(&tree_kernel<256, false, false>);
-    case 512: return reinterpret_cast<const void *>(&tree_kernel<512, false, false>);
+    case 64: return reinterpret_cast<const void *>(&tree_kernel<64, SPLIT, NET>);
+    case 128: return reinterpret_cast<const void *>(&tree_kernel<128, SPLIT, NET>);
+    case 256: return reinterpret_cast<const void *>(&tree_kernel<256, SPLIT, NET>);
+    case 512: return reinterpret_cast<const void *>(&tree_kernel<512, SPLIT, NET>);
     default: return nullptr;
     }
+}
+
+const void *tree_kernel_ptr(int tpb, bool split, bool net) {
+    if (net) return split ? nullptr : tree_kernel_of<false, true>(tpb);
+    return split ? tree_kernel_of<true, false>(tpb) : tree_kernel_of<false, false>(tpb);
 }
 
 // Channels of compartments beyond the compartment kernels' slots (more than NCH channel

@@ -73,7 +73,7 @@ __host__ __device__ inline TreeLds tree_lds(int32_t nmax, int32_t nvmax, int32_t
     L.il = L.ct + nctmax;
     L.w = (L.il + ninmax + 3) & ~3;         // task words, read up to 16 bytes at a time
     L.cx = (L.w + words_max + 3) & ~3;      // 16-byte records
-    L.gtab = L.cx + 20 * cxmax;             // 64-byte DGate records (multiple of 4 units)
+    L.gtab = L.cx + 24 * cxmax;             // 64-byte DGate records (multiple of 4 units)
     L.stab = L.gtab + 16 * n_gates;         // 32-byte DSynType records
     L.total = L.stab + 8 * n_stypes;
     return L;
