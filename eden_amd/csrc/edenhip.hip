@@ -79,6 +79,9 @@ void gate_safe_range(DGate &G, float dt) {
 struct Bucket {
     int tpb = 64;
     bool split = false;   // one extra wave runs the channel phase concurrently
+    bool lean = true;     // lean_tree_kernel runs it: every cell is TreeCell::lean
+    int64_t lean_bytes = 0;   // its largest cell's LDS there
+    const void *kernel(bool net) const { return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(tpb, split, net); }
     std::vector<int32_t> order;    // tree-cell indices, largest first
     int32_t nmax = 0;
     int32_t nvmax = 0;        // voltage slots in LDS (1 for a constant tree, else its size)
@@ -134,7 +137,7 @@ struct edenhip_ctx {
     int32_t *d_point = nullptr;
     int32_t n_point = 0;
     // tree cells
-    uint32_t *d_words = nullptr;
+    uint32_t *d_words = nullptr, *d_lean = nullptr;
     int32_t *d_pos = nullptr;
     float2 *d_u = nullptr;
     uint32_t *d_tcm = nullptr, *d_ctask = nullptr, *d_inl = nullptr, *d_gt = nullptr, *d_cflag = nullptr;
@@ -391,6 +394,99 @@ static int pool_stream(edenhip_ctx *ctx, int slot, hipStream_t *out) {
 // floats in a LEMS parameter table: the types' vectors, then any per-instance vectors
 static int64_t lems_param_count(const int32_t *param_begin, int32_t n_types, int64_t n_params) {
     return std::max<int64_t>(param_begin[n_types], n_params);
+}
+
+// The block of a lean cell (lean_tree_kernel) from its schedule: a record per task, the addresses
+// of its right-hand sides (LEAN_X + 4 p of position p, n for the dummy) and its constants.
+// D: the non-root diagonals, u: (Ui, Uj), by position. 32-bit words:
+//   directory  as plan_tree_waves's: per wave its fold and its backward list, the junction's two,
+//              each (first header / 2 | rounds << 16); then where the root's children are
+//   headers    per round, two words: the LDS address of its first record, tasks - 1
+//   records    LeanFold, LeanBwd: the schedule's words as LDS addresses (lean_tree_kernel), the
+//              ratios Uj / D' (-1 for the dummy, which holds -0), 1 / D' in double and Ui (1 and
+//              -1 for the dummy)
+//   children   per child of the root, in order, (ratio * Ui, ratio)
+// The eliminated diagonals take each node's children in ascending order, as the fold tasks do.
+// Empty where a round has no task or more than a wave's lanes.
+static std::vector<uint32_t> lean_block(const WavePlan &P, int32_t n, const int32_t *parent, int waves,
+                                        std::vector<float> &D, const float2 *u) {
+    std::vector<int32_t> par((size_t)n, -1), first((size_t)n, 0), kids((size_t)n, 0);
+    for (int32_t i = 1; i < n; i++) par[(size_t)P.pos[i]] = P.pos[parent[i]];
+    for (int32_t p = n - 1; p >= 1; p--) {   // children are consecutive positions
+        first[(size_t)par[(size_t)p]] = p;
+        kids[(size_t)par[(size_t)p]]++;
+    }
+    std::vector<float> ratio((size_t)n + 1, -1.0f), ui((size_t)n + 1, -1.0f);
+    std::vector<double> rec((size_t)n + 1, 1.0);
+    for (int32_t p = n - 1; p >= 1; p--) {
+        float x = D[(size_t)p];
+        for (int32_t c = first[(size_t)p]; c < first[(size_t)p] + kids[(size_t)p]; c++) x = x - ratio[(size_t)c] * u[c].x;
+        ratio[(size_t)p] = u[p].y / x;
+        ui[(size_t)p] = u[p].x;
+        rec[(size_t)p] = 1.0 / (double)x;
+    }
+    const std::vector<uint32_t> &S = P.block;
+    const int n_list = 2 * waves + 2;
+    const uint32_t base = LEAN_X + 4 * (uint32_t)lean_nodes(n);   // of the block
+    const int dir = (n_list + 2) / 2;                             // its directory, in pairs of words
+    int rounds = 0;
+    std::vector<uint32_t> out((size_t)dir * 2, 0u);
+    for (int l = 0; l < n_list; l++) {
+        out[(size_t)l] = (uint32_t)(dir + rounds) | (S[(size_t)l] & 0xFFFF0000u);
+        rounds += (int)(S[(size_t)l] >> 16);
+    }
+    size_t h = out.size();
+    out.resize((h + 2 * (size_t)rounds + 3) & ~(size_t)3, 0u);
+    auto fbits = [](float x) {
+        uint32_t b;
+        std::memcpy(&b, &x, 4);
+        return b;
+    };
+    auto word = [&](double x) {
+        uint64_t b;
+        std::memcpy(&b, &x, 8);
+        out.push_back((uint32_t)b);
+        out.push_back((uint32_t)(b >> 32));
+    };
+    auto node = [](uint32_t o) { return o / WAVE_NODE_BYTES; };
+    auto at = [](uint32_t p) { return LEAN_X + 4 * p; };
+    for (int l = 0; l < n_list; l++) {
+        const bool fwd = (l & 1) == 0;
+        for (uint32_t r = 0; r < S[(size_t)l] >> 16; r++) {
+            const uint32_t head = S[(S[(size_t)l] & 0xFFFFu) + r], c = head >> 16;
+            const uint32_t *w = S.data() + (head & 0xFFFFu);
+            if (c == 0 || c > 64) return {};
+            out[h++] = base + 4 * (uint32_t)out.size();
+            out[h++] = c - 1;
+            for (uint32_t k = 0; k < c; k++) {
+                if (fwd) {
+                    const uint32_t *f = w + 4 * k;
+                    const uint32_t p = node(f[0] & 0xFFFFu), c0 = node(f[0] >> 16), c1 = node(f[1] & 0xFFFFu);
+                    const uint32_t g00 = node(f[1] >> 16), g01 = node(f[2] & 0xFFFFu), g10 = node(f[2] >> 16), g11 = node(f[3]);
+                    for (uint32_t x : {c0, c1, g00, g01}) out.push_back(fbits(ratio[x]));
+                    for (uint32_t x : {c0, g00, g01, c1}) out.push_back(at(x));
+                    for (uint32_t x : {g10, g11}) out.push_back(fbits(ratio[x]));
+                    out.push_back(at(g10));
+                    out.push_back(at(g11) | at(p) << 16);
+                } else {
+                    const uint32_t p = node(w[2 * k] & 0xFFFFu), s = node(w[2 * k] >> 16), m = node(w[2 * k + 1]);
+                    word(rec[m]);
+                    out.push_back(fbits(ui[p]));
+                    out.push_back(fbits(ui[m]));
+                    word(rec[p]);
+                    out.push_back(at(s));
+                    out.push_back(at(m) | at(p) << 16);
+                }
+            }
+        }
+    }
+    out[(size_t)n_list] = (uint32_t)out.size();
+    for (int32_t c = 1; c <= kids[0]; c++) {
+        out.push_back(fbits(ratio[(size_t)c] * u[c].x));
+        out.push_back(fbits(ratio[(size_t)c]));
+    }
+    while (out.size() & 3u) out.push_back(0u);
+    return out;
 }
 
 static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
@@ -770,6 +866,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     std::vector<float> gqv;
     std::vector<uint32_t> cflag(NC, 0);
     std::vector<TreeComplex> cxv;
+    std::vector<uint32_t> lean_words;   // the lean cells' blocks (lean_block)
     std::vector<uint32_t> gtv;   // per gate variable: its channel task (local to the cell) | gate index << 16
     std::vector<int64_t> gq_first(NC, -1);   // tree compartments: index of the first gate variable in gqv
     // Hines schedules of the tree cells, planned in parallel (independent per cell); cells
@@ -914,7 +1011,27 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
             bool ok = true;
             for (int32_t i = 1; i < n && ok; i++) ok = (tcm[c0 + i] & (0xF8u | TCM_SYN | TCM_XCH)) == 0u;
             tc.const_tree = ok ? 1 : 0;
+            const bool root_cx = (cflag[c0] & TCX_COMPLEX) != 0u;
+            tc.lean = ok && tc.n_cx == (root_cx ? 1 : 0) && (tcm[c0] & (TCM_INPUT | TCM_SYN | TCM_XCH)) == 0u ? 1 : 0;
             if (ok != P.merged) return fail(ctx, EDENHIP_E_INVALID, "internal: schedule format of a constant tree");
+        }
+        if (tc.lean) {
+            // the non-root diagonals, as the kernels form them (fp32, one ungated channel)
+            std::vector<float> D((size_t)n, 0.0f);
+            for (int32_t i = 1; i < n; i++) {
+                const int64_t g = c0 + i;
+                const float G_ch = 0.0f + (((chg[g * NCH] * 1.0f) * 1e-5f) * A[g]);
+                const float G_int = (G_ch + 0.0f) + 0.0f;
+                const float Dd = 1 * (G_int / C[g]) + invrc[g];
+                D[(size_t)P.pos[i]] = 1 + Dd * d->dt;
+            }
+            const std::vector<uint32_t> blk = lean_block(P, n, d->parent + c0, tpb / 64, D, uv.data() + c0);
+            tc.lean = !blk.empty() && lean_lds((int64_t)blk.size(), n) <= 160 * 1024 - 256 ? 1 : 0;
+            if (tc.lean) {
+                tc.lean_off = (int64_t)lean_words.size();
+                tc.lean_len = (int32_t)blk.size();
+                lean_words.insert(lean_words.end(), blk.begin(), blk.end());
+            }
         }
         cells.push_back(tc);
         cell_tpb.push_back(tpb);
@@ -1269,6 +1386,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
 
     TRY(upload(ctx, &ctx->d_point, point));
     TRY(upload(ctx, &ctx->d_words, words));
+    TRY(upload(ctx, &ctx->d_lean, lean_words));
     TRY(upload(ctx, &ctx->d_pos, posv));
     TRY(upload(ctx, &ctx->d_u, uv));
     TRY(upload(ctx, &ctx->d_tcm, tcm));
@@ -1302,6 +1420,8 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         b->nctmax = std::max(b->nctmax, cells[i].n_ctask);
         b->words_max = std::max(b->words_max, cells[i].words_len);
         b->cxmax = std::max(b->cxmax, cells[i].n_cx);
+        b->lean = b->lean && cells[i].lean != 0;
+        b->lean_bytes = std::max(b->lean_bytes, lean_lds(cells[i].lean_len, cells[i].n));
     }
     // launch order: workgroups with the most waves first, so that they find whole CUs
     std::stable_sort(ctx->buckets.begin(), ctx->buckets.end(), [](const Bucket &x, const Bucket &y) { return x.tpb > y.tpb; });
@@ -1333,10 +1453,16 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         b.lds = (size_t)tree_lds(b.nmax, b.nvmax, b.ngmax, b.nctmax, b.ninmax, b.words_max, b.cxmax_lds, ctx->n_gates,
                                  ctx->n_stypes, b.split).total *
                 sizeof(float);
-        const void *kp = tree_kernel_ptr(b.tpb, b.split, ctx->tree_net);
+        // lean_tree_kernel runs a bucket of lean cells: also where its blocks, twice the LDS, leave
+        // fewer cells in flight (481 rows of 4,096 cells of up to 400 compartments 5.3 -> 4.3 ms, of
+        // up to 2,000 11.5 -> 10.9 ms)
+        b.lean = b.lean && !ctx->tree_net;
+        if (b.lean) b.lds = (size_t)b.lean_bytes;
+        const int nt = b.tpb + (b.split ? 64 : 0);
+        const void *kp = b.kernel(ctx->tree_net);
         if (!kp) return fail(ctx, EDENHIP_E_LIMIT, "no tree kernel for the chosen workgroup size");
         int per_cu = 0;
-        HIPCHECK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, b.tpb + (b.split ? 64 : 0), b.lds));
+        HIPCHECK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, nt, b.lds));
         if (per_cu <= 0) return fail(ctx, EDENHIP_E_LIMIT, "tree kernel does not fit on a CU (LDS)");
         b.grid = (int)std::min<int64_t>((int64_t)bc.size(), (int64_t)per_cu * ctx->n_cu);
         TRY(upload(ctx, &b.d_cells, bc));
@@ -1784,8 +1910,10 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 if (ctx->queue_base) args[8] = &qs[&bk - ctx->buckets.data()];
                 HIPCHECK(ctx, hipStreamWaitEvent(bk.stream, ctx->ev_start, 0));
                 if (pf && first) HIPCHECK(ctx, hipEventRecord(bk.p0, bk.stream));
-                HIPCHECK(ctx, hipLaunchKernel(tree_kernel_ptr(bk.tpb, bk.split, ctx->tree_net), dim3(bk.grid),
-                                              dim3(bk.tpb + (bk.split ? 64 : 0)), args, bk.lds, bk.stream));
+                void *largs[] = {&T, &ctx->d_gates, &bk.d_cells, &ntask, args[8], &ctx->d_lean, &ctx->d_pos, &ctx->d_gq,
+                                 (void *)&aa, (void *)&bb, &row0, &dt};
+                HIPCHECK(ctx, hipLaunchKernel(bk.kernel(ctx->tree_net), dim3(bk.grid), dim3(bk.tpb + (bk.split ? 64 : 0)),
+                                              bk.lean ? largs : args, bk.lds, bk.stream));
                 if (pf && last) HIPCHECK(ctx, hipEventRecord(bk.p1, bk.stream));
                 HIPCHECK(ctx, hipEventRecord(bk.done, bk.stream));
                 HIPCHECK(ctx, hipStreamWaitEvent(ctx->stream, bk.done, 0));

@@ -832,6 +832,352 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
     }
 }
 
+// The value at an LDS address. lean_tree_kernel has no LDS but the dynamic one, which starts at
+// address 0, so that its task records hold addresses to be used as they are.
+typedef float LdsF2 __attribute__((ext_vector_type(2)));
+typedef float LdsF4 __attribute__((ext_vector_type(4)));
+typedef uint32_t LdsU2 __attribute__((ext_vector_type(2)));
+typedef uint32_t LdsU4 __attribute__((ext_vector_type(4)));
+template <class V>
+__device__ __forceinline__ __attribute__((address_space(3))) V &lds_at(uint32_t a) {
+    return *reinterpret_cast<__attribute__((address_space(3))) V *>(a);
+}
+
+// Task records of lean_tree_kernel (lean_block). read() issues a round's reads: the values at the
+// task's addresses and the record's constants. next() reads another record's addresses in place
+// of the task's, whose own node stays in p; value() is the node's new value.
+//
+// Fold, 48 bytes: two children into a node's right-hand side; a merged child's is formed again
+// from its children (tree_kernel, fold_const). Words: the ratios of c0, c1, g00, g01; addresses
+// c0, g00, g01, c1; ratios of g10, g11, addresses g10 and (g11 | node << 16).
+struct LeanFold {
+    static constexpr uint32_t SIZE = 48;
+    uint32_t p;
+    LdsU4 a;
+    LdsU2 b;
+    float x, c0, a0, a1, c1, b0, b1;
+    LdsF4 r;
+    LdsF2 r2;
+    __device__ __forceinline__ void next(uint32_t rec) {
+        a = lds_at<LdsU4>(rec + 16);
+        b = lds_at<LdsU2>(rec + 40);
+    }
+    __device__ __forceinline__ void read(uint32_t rec) {
+        p = b.y >> 16;
+        c0 = lds_at<float>(a.x); a0 = lds_at<float>(a.y); a1 = lds_at<float>(a.z);
+        c1 = lds_at<float>(a.w); b0 = lds_at<float>(b.x); b1 = lds_at<float>(b.y & 0xFFFFu);
+        x = lds_at<float>(p);
+        r = lds_at<LdsF4>(rec);
+        r2 = lds_at<LdsF2>(rec + 32);
+    }
+    __device__ __forceinline__ float value() const {
+        const float xa = (c0 - r.z * a0) - r.w * a1;
+        const float xb = (c1 - r2.x * b0) - r2.y * b1;
+        return (x - r.x * xa) - r.y * xb;
+    }
+};
+// Backward, 32 bytes: a node from its solved parent, or from its solved grandparent through its
+// parent mid. Words: 1 / D' of mid, Ui of the node, of mid; 1 / D' of the node, addresses of the
+// solved one and (mid | node << 16). Without mid that is the dummy, with 1 / D' = 1 and Ui = -1,
+// which hands the solved voltage on.
+struct LeanBwd {
+    static constexpr uint32_t SIZE = 32;
+    uint32_t p;
+    LdsU2 a, rp;
+    LdsU4 c;
+    float x, xs, m;
+    __device__ __forceinline__ void next(uint32_t rec) {
+        a = lds_at<LdsU2>(rec + 24);
+    }
+    __device__ __forceinline__ void read(uint32_t rec) {
+        p = a.y >> 16;
+        xs = lds_at<float>(a.x); m = lds_at<float>(a.y & 0xFFFFu); x = lds_at<float>(p);
+        c = lds_at<LdsU4>(rec);
+        rp = lds_at<LdsU2>(rec + 16);
+    }
+    __device__ __forceinline__ float value() const {
+        const float xm = div_c(m - __uint_as_float(c.w) * xs, __hiloint2double((int)c.y, (int)c.x));
+        return div_c(x - __uint_as_float(c.z) * xm, __hiloint2double((int)rp.y, (int)rp.x));
+    }
+};
+
+// Cells of passive dendrites on an active soma (TreeCell::lean), as tree_kernel runs them but with
+// nothing general in the step loop, which is bound by the latency of the Hines rounds: a round is
+// one dependent trip through LDS and a short chain of operations.
+//   - Every non-root compartment's diagonal is constant, so what a round needs of it (ratios,
+//     reciprocals of eliminated diagonals, Ui) is formed on the host and lies in the round's task
+//     records (lean_block); of a node only its right-hand side, 4 bytes, is gathered. The
+//     back-substitution multiplies by the double reciprocal (div_c) where it divided.
+//   - A round first issues its gathers and the reads of its constants, behind them those of the
+//     next round's addresses, and makes the address of the record after that while they are on
+//     their way. Lanes beyond its tasks repeat the last one (the same value to the same place),
+//     so there is no execution mask to set.
+//   - The root's update, its gates, its trace and its spikes belong to the gate wave: the extra
+//     wave with SPLIT, else the last cable wave. It updates the root, down to the reciprocal of
+//     its eliminated diagonal, beside wave 0's forward rounds (the longest lists), and moves the
+//     gates beside the backward ones, both on its first quad (QuadChannels).
+// With the reading of their rows, 2,005 steps of 512 trees of up to 400 compartments 11.4 -> 5.6 ms
+// (tree_kernel, this one), 1,004 of 7 of up to 300 3.6 -> 2.0 ms; a forward round takes about 270
+// cycles, a backward one 210 (430 and 385).
+template <int TPB, bool SPLIT>
+__global__ void __launch_bounds__(TPB + (SPLIT ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(3)))
+lean_tree_kernel(DevTables T, const DGate *__restrict__ gates_g, const TreeCell *__restrict__ cells,
+                 int32_t n_tasks, int32_t *__restrict__ queue, const uint32_t *__restrict__ blocks_g,
+                 const int32_t *__restrict__ pos_g, float *__restrict__ gq_g, int64_t s0, int64_t s1, int64_t row0,
+                 float dt) {
+    constexpr int K = TREE_SLOTS, W = TPB / 64, NT = TPB + (SPLIT ? 64 : 0);
+    // the cell's number, its root's voltage at the start of the step, right-hand side and the
+    // reciprocal of its eliminated diagonal, then (LEAN_X) the right-hand sides by position: the
+    // dummy at N is -0, which folds with ratio -1 leave as it is, N + 1 takes what nobody reads
+    constexpr uint32_t AT_TASK = 0, AT_V = 4, AT_R = 8, AT_RHS = 16;
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    const bool cable = !SPLIT || tid < TPB;
+    const bool gate_wave = SPLIT ? !cable : wv == W - 1;
+    auto X = [](uint32_t o) -> auto & { return lds_at<float>(o); };
+    for (;;) {
+        __syncthreads();
+        if (tid == 0) lds_at<int32_t>(AT_TASK) = atomicAdd(&queue[0], 1);
+        __syncthreads();
+        const int32_t task = lds_at<int32_t>(AT_TASK);
+        if (task >= n_tasks) break;
+        const TreeCell cell = cells[task];
+        const int32_t N = cell.n;
+        const int64_t c0 = cell.comp_begin, gq0 = cell.gate_off;
+        const uint32_t blk = LEAN_X + 4u * (uint32_t)lean_nodes(N);
+        const uint4 *const bg = reinterpret_cast<const uint4 *>(blocks_g + cell.lean_off);
+        for (int i = tid; i < cell.lean_len / 4; i += NT) {
+            const uint4 w = bg[i];
+            lds_at<LdsU4>(blk + 16u * (uint32_t)i) = LdsU4{w.x, w.y, w.z, w.w};
+        }
+        if (tid == 0) {
+            X(LEAN_X + 4 * N) = -0.0f;
+            lds_at<float>(AT_V) = T.V[c0];
+        }
+        // cable slots: voltage, channel, area, conductance sum, 1 / C and position, as in
+        // tree_kernel; the root's and those beyond the cell write to N + 1
+        float V[K], g0[K], e0[K], Ar[K], Gs[K];
+        double rC[K];
+        uint32_t po[K];
+        const int slots = (N - (tid & ~63) + TPB - 1) / TPB;     // of the wave
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            const int c = tid + TPB * j;
+            V[j] = 0.0f; g0[j] = 0.0f; e0[j] = 0.0f; Ar[j] = 0.0f; Gs[j] = 0.0f; rC[j] = 1.0;
+            po[j] = LEAN_X + 4u * (uint32_t)N + 4u;
+            if (cable && c < N && c > 0) {
+                const int64_t g = c0 + c;
+                po[j] = LEAN_X + 4u * (uint32_t)pos_g[g];
+                V[j] = T.V[g];
+                g0[j] = T.chg[g * NCH];
+                e0[j] = T.che[g * NCH];
+                Ar[j] = T.A[g];
+                rC[j] = 1.0 / (double)T.C[g];
+                const float G_ch = 0.0f + (((g0[j] * 1.0f) * 1e-5f) * Ar[j]);
+                Gs[j] = (G_ch + 0.0f) + 0.0f;
+            }
+        }
+        // gate wave: the root's constants and gate variable lane & 3
+        QuadChannels ch;
+        CompConst k;
+        float qv = 0.0f;
+        double root_rC = 1.0;
+        const int qs = lane & 3;
+        if (gate_wave) {
+            load_comp_const(T, c0, k);
+            ch.load(gates_g, k, qs);
+            root_rC = 1.0 / (double)k.C;
+            if (qs < cell.n_gate) qv = gq_g[gq0 + qs];
+        }
+        __syncthreads();
+        // a list: its rounds' headers (two words: the address of the first record, tasks - 1), a
+        // lane each for the first 64, the last one repeated
+        struct List {
+            int first, cnt;
+            LdsU2 h;
+        };
+        auto dir = [&](int i) { return (uint32_t)__builtin_amdgcn_readfirstlane(lds_at<uint32_t>(blk + 4u * (uint32_t)i)); };
+        auto headers = [&](const List &L, int r) {
+            const uint32_t at = blk + 8u * (uint32_t)(L.first + min(r + lane, L.cnt - 1));
+            return (LdsU2)lds_at<LdsU2>(at);
+        };
+        auto load_list = [&](int i) {
+            List L;
+            const uint32_t e = dir(i);
+            L.first = e & 0xFFFFu;
+            L.cnt = e >> 16;
+            L.h = LdsU2{0u, 0u};
+            if (L.cnt > 0) L.h = headers(L, 0);
+            return L;
+        };
+        const int lw = cable ? wv : 0;
+        const List Lf = load_list(2 * lw), Lb = load_list(2 * lw + 1);
+        const List Ljf = load_list(2 * W), Ljb = load_list(2 * W + 1);
+        // the root's first 64 children (positions 1 .. nr), a lane each: ratio * Ui and ratio,
+        // both 0 beyond them
+        const int nr = cell.root_children;
+        const uint32_t kids = blk + 4u * dir(2 * W + 2);
+        auto kid_at = [&](int i) { return (LdsF2)lds_at<LdsF2>(kids + 8u * (uint32_t)i); };
+        LdsF2 kid = {0.0f, 0.0f};
+        if (lane < nr) kid = kid_at(lane);
+        const uint32_t kid_x = LEAN_X + 4u * (uint32_t)(lane < nr ? 1 + lane : N);
+        // a - v[0] - v[1] ... over the lanes' values, in order
+        auto minus_lanes = [](float a, float v, int n) {
+            for (int i = 0; i < n; i += 4) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    a = a - __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i + j));
+            }
+            return a;
+        };
+        // the record of a lane's task in the round with header r of h
+        auto record = [&](LdsU2 h, int r, uint32_t size) -> uint32_t {
+            const uint32_t n = (uint32_t)__builtin_amdgcn_readlane(h.y, r);
+            return (uint32_t)__builtin_amdgcn_readlane(h.x, r) + __umul24(min((uint32_t)lane, n), size);
+        };
+        // a list about to run: its first round's record and addresses
+        auto begin = [&](const List &L, auto &t, uint32_t &rec) {
+            if (L.cnt == 0) return;
+            rec = record(L.h, 0, t.SIZE);
+            t.next(rec);
+        };
+        // Round after round with no barrier, as in tree_kernel
+        auto run_list = [&](const List &L, auto t, uint32_t rec) {
+            LdsU2 h = L.h;
+            for (int r0 = 0; r0 < L.cnt; r0 += 63) {
+                if (r0 > 0) h = headers(L, r0);
+                const int n = __builtin_amdgcn_readfirstlane(min(63, L.cnt - r0));
+                for (int r = 1; r <= n; r++) {
+                    t.read(rec);
+                    rec = record(h, r, t.SIZE);
+                    __builtin_amdgcn_sched_barrier(0);
+                    t.next(rec);
+                    __builtin_amdgcn_sched_barrier(0);
+                    X(t.p) = t.value();
+                }
+            }
+        };
+        auto barrier_all = [] {
+            if constexpr (NT > 64)
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else
+                lds_barrier<64>();
+        };
+        float Vr = 0.0f;           // the root's voltage (gate wave)
+        double time = (s0 >= 1) ? T.t_row[s0 - 1] : 0.0;
+        for (int64_t s = s0; s < s1; s++) {
+            const bool init = s <= 0;
+            const float t = (float)time;
+            if (!init) time += (double)dt;
+            if (gate_wave) {
+                // the spike of the step before, this step's trace row
+                const float Vp = Vr;
+                Vr = lds_at<float>(AT_V);
+                if (s > s0 && Vp < k.vthr && k.vthr < Vr && lane == 0) log_event(T, k.ev, s - 1);
+                if (!init && k.rec >= 0 && lane == 0) trace_at(T, k.rec, s - 1 - row0) = Vr;
+            }
+            if (!init) {
+                LeanFold tf{};
+                LeanBwd tb{};
+                uint32_t rf = 0, rb = 0;     // their records
+                if (cable) {
+#pragma unroll
+                    for (int j = 0; j < K; j++) {
+                        if (j >= 2 && j >= slots) continue;
+                        const float I_ch = 0.0f + ((((g0[j] * 1.0f) * (e0[j] - V[j])) * 1e-5f) * Ar[j]);
+                        const float I_int = (I_ch + 0.0f) + 0.0f;
+                        X(po[j]) = V[j] + div_c(dt * (I_int + ((V[j] * Gs[j]))), rC[j]);
+                    }
+                    begin(Lf, tf, rf);
+                }
+                if constexpr (TPB > 64) barrier_all();
+                else lds_barrier<64>();
+                if (gate_wave) {
+                    float I_ch, G_ch;
+                    ch.currents(qv, Vr, I_ch, G_ch);
+                    const float I_in = pulses_current(T, k, c0, t), G_in = 0.0f;
+                    const float I_syn = 0.0f, G_syn = 0.0f;
+                    const float I_int = I_ch + I_in + I_syn;
+                    const float G_int = G_ch + G_in + G_syn;
+                    const float Dd = 1 * div_c(G_int, root_rC) + k.invrc;
+                    const float x = Vr + div_c(dt * (I_int + ((Vr * G_int))), root_rC);
+                    float D = minus_lanes(1 + Dd * dt, kid.x, min(nr, 64));
+                    for (int b = 64; b < nr; b += 64)
+                        D = minus_lanes(D, b + lane < nr ? kid_at(b + lane).x : 0.0f,
+                                        min(nr - b, 64));
+                    double r = recip64(D);
+                    const float ad = fabsf(D);
+                    if (__builtin_expect(!((ad >= 0x1p-60f) & (ad <= 0x1p60f)), 0)) r = 1.0 / (double)D;
+                    if (lane == 0) {
+                        lds_at<float>(AT_RHS) = x;
+                        lds_at<double>(AT_R) = r;
+                    }
+                }
+                if (cable) {
+                    run_list(Lf, tf, rf);
+                    begin(Lb, tb, rb);
+                }
+                barrier_all();      // forward lists and the root's update done
+                if (wv == 0) {
+                    if (Ljf.cnt > 0) {
+                        begin(Ljf, tf, rf);
+                        run_list(Ljf, tf, rf);
+                    }
+                    float x = minus_lanes(lds_at<float>(AT_RHS), kid.y * X(kid_x), min(nr, 64));
+                    for (int b = 64; b < nr; b += 64)
+                        x = minus_lanes(x, b + lane < nr ? kid_at(b + lane).y *
+                                                               X(LEAN_X + 4u * (uint32_t)(1 + b + lane))
+                                                         : 0.0f,
+                                        min(nr - b, 64));
+                    x = div_c(x, lds_at<double>(AT_R));
+                    if (lane == 0) {
+                        X(LEAN_X) = x;
+                        lds_at<float>(AT_V) = x;
+                    }
+                    lds_barrier<64>();
+                    if (Ljb.cnt > 0) {
+                        LeanBwd tj{};
+                        begin(Ljb, tj, rf);
+                        run_list(Ljb, tj, rf);
+                    }
+                }
+                if constexpr (TPB > 64) barrier_all();
+                if (cable) run_list(Lb, tb, rb);
+            }
+            if (gate_wave) qv = ch.next(qv, Vr, init, dt);
+            if constexpr (TPB > 64)
+                if (!init) barrier_all();       // every node solved
+            if (cable && !init) {
+#pragma unroll
+                for (int j = 0; j < K; j++) V[j] = X(po[j]);
+            }
+            // (the next step starts with a lane's own right-hand sides; the root's voltage was
+            // written before the junction's barrier, or, with one cable wave, by this one)
+            if constexpr (TPB == 64 && SPLIT) barrier_all();
+        }
+        if (gate_wave) {
+            const float Vn = lds_at<float>(AT_V);
+            if (Vr < k.vthr && k.vthr < Vn && lane == 0) log_event(T, k.ev, s1 - 1);
+            if (lane == 0) T.V[c0] = Vn;
+            if (lane < cell.n_gate) gq_g[gq0 + lane] = qv;
+        }
+        if (cable) {
+#pragma unroll
+            for (int j = 0; j < K; j++) {
+                const int c = tid + TPB * j;
+                if (c < N && c > 0) T.V[c0 + c] = V[j];
+            }
+        }
+    }
+    // the last workgroup out resets the queue for the next launch
+    if (tid == 0) {
+        __threadfence();
+        if (atomicAdd(&queue[1], 1) == (int)gridDim.x - 1) {
+            queue[0] = 0;
+            queue[1] = 0;
+        }
+    }
+}
+
 template <bool SPLIT, bool NET>
 static const void *tree_kernel_of(int tpb) {
     switch (tpb) {
@@ -843,9 +1189,24 @@ static const void *tree_kernel_of(int tpb) {
     }
 }
 
+template <bool SPLIT>
+static const void *lean_kernel_of(int tpb) {
+    switch (tpb) {
+    case 64: return reinterpret_cast<const void *>(&lean_tree_kernel<64, SPLIT>);
+    case 128: return reinterpret_cast<const void *>(&lean_tree_kernel<128, SPLIT>);
+    case 256: return reinterpret_cast<const void *>(&lean_tree_kernel<256, SPLIT>);
+    case 512: return reinterpret_cast<const void *>(&lean_tree_kernel<512, SPLIT>);
+    default: return nullptr;
+    }
+}
+
 const void *tree_kernel_ptr(int tpb, bool split, bool net) {
     if (net) return split ? nullptr : tree_kernel_of<false, true>(tpb);
     return split ? tree_kernel_of<true, false>(tpb) : tree_kernel_of<false, false>(tpb);
+}
+
+const void *lean_tree_kernel_ptr(int tpb, bool split) {
+    return split ? lean_kernel_of<true>(tpb) : lean_kernel_of<false>(tpb);
 }
 
 // Channels of compartments beyond the compartment kernels' slots (more than NCH channel

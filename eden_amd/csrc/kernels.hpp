@@ -25,6 +25,10 @@ struct TreeCell {
     int32_t cx_off;       // offset of their records
     int32_t const_tree;   // 1: constant diagonals below the root (see tree_kernel)
     int32_t root_children;   // children of the root (BFS positions 1 .. root_children)
+    int32_t lean;         // 1: a constant tree with no complex compartment but a root without
+                          // inputs, synapses or channels of another pass (lean_tree_kernel)
+    int32_t lean_len;     // its lean block, 32-bit words (a multiple of 4)
+    int64_t lean_off;     // where it starts
 };
 
 // Per-compartment flag word of tree cells: 0 for a simple compartment (one ungated channel,
@@ -131,6 +135,13 @@ constexpr int NET_QUAD_MAX = 16;
 // net: the variant for networks (synapses on tree compartments, spikes sent to recipients),
 // launched one step at a time; only without a channel wave.
 const void *tree_kernel_ptr(int tpb, bool split, bool net = false);
+// for buckets whose cells are all TreeCell::lean
+const void *lean_tree_kernel_ptr(int tpb, bool split);
+// Dynamic LDS of lean_tree_kernel: a few scalars, from LEAN_X on the right-hand sides (two more
+// than nodes), then the cell's block, all multiples of 16 bytes.
+constexpr uint32_t LEAN_X = 32;
+__host__ __device__ inline int64_t lean_nodes(int64_t n) { return (n + 2 + 3) & ~(int64_t)3; }
+inline int64_t lean_lds(int64_t lean_len, int64_t n) { return LEAN_X + 4 * (lean_nodes(n) + lean_len); }
 const void *net_window_kernel_ptr();
 const void *net_quad_kernel_ptr(int groups);
 const void *net_deliver_kernel_ptr();

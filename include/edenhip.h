@@ -421,7 +421,9 @@ int edenhip_kernel_stats(const edenhip_ctx *ctx, double *total_ms, int64_t *laun
  * the chunks run since create or reset, the time from the event recorded before the
  * kernel's first launch in a chunk to the event after its last, on the kernel's stream. */
 typedef struct edenhip_kernel_info {
-    char name[64];               /* kernel name as a profiler lists it, without arguments */
+    char name[64];               /* kernel name as a profiler lists it, without arguments (tree
+                                    cells: always the general kernel's, also where
+                                    lean_tree_kernel runs them) */
     int32_t threads_per_block;
     int32_t grid;                /* workgroups per launch */
     int32_t n_cells;             /* cells this kernel advances */
