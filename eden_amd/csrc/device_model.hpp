@@ -111,6 +111,9 @@ struct DevTables {
                             // ext_channels_kernel (chmeta == CHM_EXTERNAL), or null
 };
 
+// lems_syn_kernel's workgroup: compartments, and at most so many instances of each at a time.
+constexpr int LEMS_SYN_COMPS = 16, LEMS_SYN_LANES = 32;
+
 // Arguments of lems_syn_kernel (the generic LEMS synapse kernel, compiled at run time from
 // lems_kernel.hip): shared by that compilation and the host code that launches it.
 struct LemsArgs {

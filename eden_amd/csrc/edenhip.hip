@@ -191,6 +191,7 @@ struct edenhip_ctx {
     std::vector<void *> allocs;
     // generic LEMS synapses: the run-time compiled synapse kernel and its tables
     hipFunction_t lems_fn = nullptr;
+    int32_t lems_threads = 64;    // of a workgroup of lems_syn_kernel
     int32_t *d_lems_comps = nullptr;
     int32_t n_lems_comps = 0;
     float *d_lems_params = nullptr, *d_lems_state = nullptr;
@@ -1205,6 +1206,11 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         for (int64_t g = 0; g < NC; g++)
             if (syn_cnt[g] > 0) lc.push_back((int32_t)g);
         ctx->n_lems_comps = (int32_t)lc.size();
+        // lanes for the most instances of a compartment, a power of two; whole waves
+        int32_t most = 0, lanes = 64 / LEMS_SYN_COMPS;
+        for (int32_t g : lc) most = std::max(most, syn_cnt[g]);
+        while (lanes < most && lanes < LEMS_SYN_LANES) lanes *= 2;
+        ctx->lems_threads = LEMS_SYN_COMPS * lanes;
         int32_t smax = 1;
         for (int t = 0; t < LS->n_types; t++) smax = std::max(smax, LS->n_state[t]);
         const int64_t np = lems_param_count(LS->param_begin, LS->n_types, d->abi_version >= 4 ? LS->n_params : 0);
@@ -1847,8 +1853,8 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 int64_t st = a;
                 float dt = ctx->dt;
                 void *args[] = {&T, &la, &st, &dt};
-                HIPCHECK(ctx, hipModuleLaunchKernel(ctx->lems_fn, (unsigned)((ctx->n_lems_comps + 63) / 64), 1, 1, 64, 1, 1,
-                                                    0, ctx->stream, args, nullptr));
+                HIPCHECK(ctx, hipModuleLaunchKernel(ctx->lems_fn, (unsigned)((ctx->n_lems_comps + LEMS_SYN_COMPS - 1) / LEMS_SYN_COMPS),
+                                                    1, 1, (unsigned)ctx->lems_threads, 1, 1, 0, ctx->stream, args, nullptr));
                 nl++;
             }
             if (ctx->lems_cell_fn && ctx->n_acells > 0) {

@@ -70,9 +70,10 @@ int rtc_lems_kernel(const std::string &generated, hipFunction_t *fn, hipFunction
     }
     const std::string off = "--offload-arch=" + arch;
     // the same floating-point settings as the library's own kernels: no contraction, IEEE
-    // division and square root
-    const char *opts[] = {off.c_str(), "-O3", "-std=c++17", "-ffp-contract=off", "-fno-fast-math"};
-    const hiprtcResult rc = hiprtcCompileProgram(prog, 5, opts);
+    // division and square root, no packed fp32 operations
+    const char *opts[] = {off.c_str(),       "-O3",     "-std=c++17",      "-ffp-contract=off", "-fno-fast-math",
+                          "-Xclang",         "-target-feature", "-Xclang", "-packed-fp32-ops"};
+    const hiprtcResult rc = hiprtcCompileProgram(prog, 9, opts);
     if (rc != HIPRTC_SUCCESS) {
         size_t n = 0;
         hiprtcGetProgramLogSize(prog, &n);

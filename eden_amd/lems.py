@@ -636,6 +636,25 @@ def _emit_assign(L, assigns, names, indent):
         L.append(f"{indent}s_{s_} = {infix(parse(expr), names)}; n_{s_} = s_{s_};")
 
 
+def _symbols(tree):
+    """Names an expression tree reads."""
+    if tree[0] == "sym":
+        return {tree[1]}
+    return set().union(*(_symbols(x) for x in tree[1:] if isinstance(x, tuple)))
+
+
+def _event_only(st):
+    """The derived parameters that nothing but an event's assignments reads."""
+    texts = [e for _, v in st.derived for e in ([v] if isinstance(v, str) else [x for case in v for x in case])]
+    texts += list(st.derivatives.values()) + list(st.on_start.values())
+    texts += [x for test, assigns in st.on_conditions for x in [test] + [e for _, e in assigns]]
+    used = {st.expose_i, st.expose_g}.union(*(_symbols(parse(x)) for x in texts if x is not None))
+    for d, expr in reversed(st.derived_params):
+        if d in used:
+            used |= _symbols(parse(expr))
+    return {d for d, _ in st.derived_params if d not in used}
+
+
 def emit(name, st, fn_name, dialect):
     """C / HIP text of one type's step function:
 
@@ -661,9 +680,13 @@ def emit(name, st, fn_name, dialect):
     for c, val in st.constants:
         L.append(f"    const float c_{c} = {_lit(val)};")
         names[c] = f"c_{c}"
+    # (what only an event needs, an expTwoSynapse's logarithm and exponentials, is formed there
+    # and not at every step)
+    late = _event_only(st)
     for d, expr in st.derived_params:
-        L.append(f"    const float dp_{d} = {infix(parse(expr), names)};")
-        names[d] = f"dp_{d}"
+        if d not in late:
+            L.append(f"    const float dp_{d} = {infix(parse(expr), names)};")
+            names[d] = f"dp_{d}"
     for k, s_ in enumerate(st.state):
         L.append(f"    float s_{s_} = S[{k} * stride];")
         names[s_] = f"s_{s_}"
@@ -683,6 +706,10 @@ def emit(name, st, fn_name, dialect):
         _emit_assign(L, assigns, names, "            ")
         L.append("        }")
     L.append("        if (event) {")
+    for d, expr in st.derived_params:
+        if d in late:
+            L.append(f"            const float dp_{d} = {infix(parse(expr), names)};")
+            names[d] = f"dp_{d}"
     _emit_assign(L, st.on_event.items(), names, "            ")
     L.append("        }")
     L.append("    }")
