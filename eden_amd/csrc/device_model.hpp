@@ -75,6 +75,9 @@ struct DevTables {
     const float *syn_weight, *syn_delay;
     float *syn_next, *syn_A, *syn_B;   // state
     int32_t *trig[2];                  // trigger flags, double-buffered
+    // per synapse slot: spikes sent to it by step of the running launch (bit i: by its step i,
+    // read at step i + 1), applied by trig_fold_kernel after it; null: launches of one step
+    unsigned long long *trig_mask;
     const int32_t *spk_begin;          // [NC+1]
     const int32_t *spk_target;
     // Poisson inputs (CSR over compartments)
@@ -263,9 +266,14 @@ __device__ __forceinline__ void log_event(const DevTables &T, int32_t col, int64
     }
 }
 
-// A spike of compartment gidx sets its recipients' trigger flags for the next step.
-__device__ __forceinline__ void send_spike(const DevTables &T, int64_t gidx, int nxt) {
+// A spike of compartment gidx sets its recipients' trigger flags for the next step, or, where
+// several steps run in a launch, their bits for that step (the launch's step number `at`).
+__device__ __forceinline__ void send_spike(const DevTables &T, int64_t gidx, int nxt, int at = 0) {
     const int32_t b = T.spk_begin[gidx], e = T.spk_begin[gidx + 1];
+    if (T.trig_mask) {
+        for (int32_t k = b; k < e; k++) atomicOr(&T.trig_mask[T.spk_target[k]], 1ull << at);
+        return;
+    }
     int32_t *trig = T.trig[nxt];
     for (int32_t k = b; k < e; k++) trig[T.spk_target[k]] = 1;   // idempotent flag (EDEN: atomic OR 1)
 }
@@ -501,6 +509,7 @@ struct CompConst {
 struct alignas(16) TreeComplex {
     CompConst k;
     uint32_t tcm;
+    int32_t syn_base, syn_cnt;   // T.syn_base, T.syn_cnt
     double rC;      // 1 / C (div_c)
 };
 static_assert(sizeof(TreeComplex) == 96, "TreeComplex layout");
@@ -736,8 +745,8 @@ __device__ __forceinline__ void exptwo_step(const DSynType &st, float V, float &
 // expTwo dynamics, per-type aggregation in list order (eden/Eden.cpp:3636-3740). The fields
 // of SYN_CHUNK synapses are loaded before any of them is computed (independent loads in
 // flight); the accumulation stays sequential in synapse order.
-constexpr int SYN_CHUNK = 8;
-
+// A point cell has many, a tree's compartment mostly one or two: 8 and 2 at a time.
+template <int SYN_CHUNK>
 __device__ __forceinline__ void synapses_step(const DevTables &T, const DSynType *__restrict__ stypes, int32_t base,
                                               int32_t cnt, float V, bool init, float t, float dt, int now,
                                               int64_t step, float &I_syn, float &G_syn) {

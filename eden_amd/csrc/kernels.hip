@@ -62,7 +62,7 @@ point_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const 
                 I_syn = e.x;
                 G_syn = e.y;
             } else {
-                synapses_step(T, stypes, syn_base, syn_cnt, V, init, t, dt, now, s, I_syn, G_syn);
+                synapses_step<8>(T, stypes, syn_base, syn_cnt, V, init, t, dt, now, s, I_syn, G_syn);
             }
         }
         float I_in = pulses_current(T, k, g, t), G_in = 0.0f;
@@ -87,7 +87,7 @@ point_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const 
             Vn = Vn / D;
         }
         if (V < k.vthr && k.vthr < Vn) {
-            if (has_spk) send_spike(T, g, nxt);
+            if (has_spk) send_spike(T, g, nxt, (int)(s - s0));
             log_event(T, k.ev, s);
         }
         V = Vn;
@@ -234,7 +234,8 @@ __device__ __forceinline__ void channel_phase(const DGate *gates, const uint32_t
 // takes its header from a lane, reads everything before its first use and divides by constants
 // through double (div_c); the root's update runs its channels on a quad (QuadChannels). 7 trees of up
 // to 300 compartments, 1,004 steps and their rows read: 4.1 -> 3.6 ms.
-// NET: networks, launched one step at a time. A compartment with chemical synapses
+// NET: networks, launched for a window of steps shorter than every delay (see trig_fold_kernel),
+// else one step at a time. A compartment with chemical synapses
 // (TCM_SYN) runs them in its complex update, with the trigger flags of the step's parity as
 // the point kernel does, and a compartment with spike recipients sends its spikes to the
 // next step's flags; both are complex compartments, so the per-slot code of the other
@@ -532,8 +533,8 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                             G_in += e2.y;
                         }
                     } else {
-                        synapses_step(T, stypes, T.syn_base[g], T.syn_cnt[g], V[j], init, t, dt, (int)((s + 3) & 1), s,
-                                      I_syn, G_syn);
+                        synapses_step<2>(T, stypes, cx.syn_base, cx.syn_cnt, V[j], init, t, dt, (int)((s + 3) & 1), s,
+                                         I_syn, G_syn);
                     }
                 }
             }
@@ -796,7 +797,7 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                             const float vthr = cx.k.vthr;
                             if (V[j] < vthr && vthr < Vn[j]) {
                                 log_event(T, cx.k.ev, s);
-                                if constexpr (NET) send_spike(T, c0 + c, (int)((s + 3) & 1) ^ 1);
+                                if constexpr (NET) send_spike(T, c0 + c, (int)((s + 3) & 1) ^ 1, (int)(s - s0));
                             }
                         }
                         V[j] = Vn[j];

@@ -326,7 +326,9 @@ typedef struct edenhip_options {
     int32_t network_window;       /* networks of one-compartment cells: 0 = advance cells several
                                      steps per launch (up to the minimum delay) with ring-buffer
                                      delivery; -1 = one launch per step; -2 = windows, each run
-                                     again step by step (exercises the exact fallback) */
+                                     again step by step (exercises the exact fallback). Networks
+                                     with multi-compartment cells: 0 = several steps per launch
+                                     where delays allow it, else one */
     int32_t size_limits[4];       /* largest tree cell (compartments) given 64, 128, 256 and
                                      512 threads; all 0 = 256, 512, 1024, 2047. A cell takes
                                      the first size whose limit holds it (each limit at most 4
