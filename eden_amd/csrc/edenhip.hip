@@ -126,6 +126,7 @@ struct edenhip_ctx {
     int32_t *d_grec_col = nullptr;
     int64_t *d_grec_src = nullptr;
     int32_t n_grec = 0;
+    bool grec_other = false;      // some are not point neurons' state variables
     std::vector<std::vector<int64_t>> ev_expand;   // dev event column -> desc columns
     int64_t chunk_rows = 0, last_row0 = 0, last_rows = 0;
     DevTables T{};
@@ -154,6 +155,7 @@ struct edenhip_ctx {
         int64_t launches;
     };
     std::vector<GraphEntry> graphs;
+    int32_t window_opt = 0;       // options.network_window as given, -1 with launches of one step
     int32_t step_window = 1;      // steps per launch of the general network path (trig_fold_kernel)
     int n_cu = 256;
     // initial copies of the state tables (for edenhip_reset)
@@ -225,6 +227,9 @@ struct edenhip_ctx {
     float2 *d_inp_ext = nullptr;         // per compartment: the LEMS inputs' (I, G) of the step
     // LEMS point neurons: the run-time compiled cell kernel and its tables (one slot per cell)
     hipFunction_t lems_cell_fn = nullptr;
+    hipFunction_t lems_window_fn = nullptr;    // null: launches of one step
+    // recorded state variables of point neuron i: [begin[i], begin[i + 1]) of (variable, column)
+    int32_t *d_arec_begin = nullptr, *d_arec_var = nullptr, *d_arec_col = nullptr;
     int32_t n_acells = 0;
     int32_t *d_acell_comps = nullptr, *d_acell_type = nullptr, *d_acell_pbegin = nullptr, *d_acell_vstate = nullptr;
     float *d_acell_params = nullptr, *d_acell_state = nullptr;
@@ -871,6 +876,8 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     }
     ctx->n_dev_cols += (int32_t)grec.size();
     // state read back between launches: recorded gate variables need one launch per step
+    // (but for point neurons' state variables, which lems_window_kernel records: build_step_window)
+    ctx->window_opt = ctx->opt.persistent < 0 ? -1 : ctx->opt.network_window;
     if (!grec.empty()) {
         ctx->opt.persistent = -1;
         ctx->opt.network_window = -1;
@@ -1191,6 +1198,26 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
             grec_src[k] = g * NQ + j;
     }
     ctx->n_grec = (int32_t)grec.size();
+    if (ctx->n_acells > 0) {
+        // the same by point neuron
+        std::vector<int32_t> begin((size_t)ctx->n_acells + 1, 0), var, col;
+        for (const auto &r : grec)
+            if (acell_slot[r.first] >= 0) begin[(size_t)acell_slot[r.first] + 1]++;
+            else ctx->grec_other = true;
+        for (size_t i = 1; i < begin.size(); i++) begin[i] += begin[i - 1];
+        var.resize((size_t)begin.back());
+        col.resize(var.size());
+        std::vector<int32_t> at(begin.begin(), begin.end() - 1);
+        for (size_t k = 0; k < grec.size(); k++)
+            if (acell_slot[grec[k].first] >= 0) {
+                const size_t p = (size_t)at[(size_t)acell_slot[grec[k].first]]++;
+                var[p] = (int32_t)grec[k].second;
+                col[p] = grec_col[k];
+            }
+        TRY(upload(ctx, &ctx->d_arec_begin, begin));
+        TRY(upload(ctx, &ctx->d_arec_var, var));
+        TRY(upload(ctx, &ctx->d_arec_col, col));
+    }
     if (ctx->n_grec > 0) {
         TRY(upload(ctx, &ctx->d_grec_col, grec_col));
         TRY(upload(ctx, &ctx->d_grec_src, grec_src));
@@ -1333,17 +1360,22 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
                                              "float *, long, float, float, float, int, int, float, float *i, float *g) "
                                              "{ *i = 0.0f; *g = 0.0f; }\n");
         gen += "\n";
-        gen += LC ? std::string(LC->source)
-                  : std::string("__device__ __forceinline__ void lems_cell(int, const float *, const float *, float *, "
-                                "long, float, float, int, float, int, long long, int *spike) { *spike = 0; }\n");
+        if (LC) gen += LC->source;
         gen += "\n";
         gen += rates_src ? std::string(rates_src)
                          : std::string("__device__ float lems_rate(int, float) { return 0.0f; }\n");
+        // lems_window_kernel: only point neurons have generic synapses, none a peer
+        bool window = ctx->n_acells > 0 && !ctx->grec_other;
+        for (int64_t g = 0; g < NC && window && lems; g++) window = syn_cnt[g] == 0 || acell_slot[g] >= 0;
+        for (int64_t k = 0; k < n_syn && window && lems && d->abi_version >= 3 && LS->peer; k++) window = LS->peer[k] < 0;
+        if (window) TRY(build_step_window(ctx, d));
+        const int kernels = ctx->step_window > 1 ? 3 : ctx->n_acells > 0 ? 2 : lems && n_syn > 0 ? 1 : 0;
         std::string err;
-        hipFunction_t syn_fn = nullptr, cell_fn = nullptr, ext_fn = nullptr;
-        if (rtc_lems_kernel(gen, &syn_fn, &cell_fn, &ext_fn, err) != 0) return fail(ctx, EDENHIP_E_INVALID, err);
+        hipFunction_t syn_fn = nullptr, cell_fn = nullptr, ext_fn = nullptr, window_fn = nullptr;
+        if (rtc_lems_kernel(gen, kernels, &syn_fn, &cell_fn, &ext_fn, &window_fn, err) != 0) return fail(ctx, EDENHIP_E_INVALID, err);
         if (lems && n_syn > 0) ctx->lems_fn = syn_fn;
         if (ctx->n_acells > 0) ctx->lems_cell_fn = cell_fn;
+        ctx->lems_window_fn = window_fn;
         if (rates_rtc) ctx->ext_rtc_fn = ext_fn;
     }
     if (ctx->n_acells > 0) {
@@ -1537,7 +1569,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     }
     HIPCHECK(ctx, hipEventCreateWithFlags(&ctx->ev_start, hipEventDisableTiming));
     TRY(build_netwin(ctx, d, point, st));
-    TRY(build_step_window(ctx, d));
+    if (!ctx->netwin && !lems && ctx->n_acells == 0 && ctx->n_grec == 0) TRY(build_step_window(ctx, d));
     TRY(upload(ctx, &ctx->d_snaps, ctx->snaps));
     for (const auto &sn : ctx->snaps) ctx->snap_max = std::max(ctx->snap_max, (int64_t)sn.bytes);
     if (!ctx->desc_to_dev_col.empty()) {
@@ -1562,19 +1594,17 @@ static bool step_windows_overlap(const edenhip_model_desc *d) {
     return false;
 }
 
-// The general network path: how many steps a launch may run (trig_fold_kernel). Generic synapses,
-// point neurons, channel pre-passes and recorded gate variables have kernels of their own between
-// the steps, and keep launches of one.
+// The general network path: how many steps a launch may run (trig_fold_kernel). Generic synapses
+// and point neurons that lems_window_kernel does not take, channel pre-passes and other recorded
+// state have kernels of their own between the steps, and keep launches of one.
 static int build_step_window(edenhip_ctx *ctx, const edenhip_model_desc *d) {
-    const int32_t nw = ctx->opt.network_window;
-    if (!ctx->network || ctx->netwin || ctx->opt.persistent < 0 || nw < 0 || ctx->lems_fn || ctx->n_acells > 0 ||
-        ctx->n_xcomp > 0 || ctx->n_grec > 0 || ctx->T.syn_ext || step_windows_overlap(d))
-        return 0;
+    const int32_t nw = ctx->window_opt;
+    if (!ctx->network || nw < 0 || ctx->n_xcomp > 0 || step_windows_overlap(d)) return 0;
     double dmin = INFINITY;
     for (int64_t k = 0; k < d->comp_spike_begin[d->n_comps]; k++)
         dmin = std::min(dmin, (double)d->syn_delay[d->spike_target[k]]);
-    if (!(dmin < INFINITY)) return 0;
-    const int64_t W = std::min<int64_t>(nw > 0 ? std::min(nw, 64) : 64, (int64_t)std::floor(dmin / (double)d->dt) - 2);
+    const double most = std::min(64.0, std::floor(dmin / (double)d->dt) - 2.0);
+    const int64_t W = nw > 0 ? std::min<int64_t>(nw, (int64_t)most) : (int64_t)most;
     if (W < 2) return 0;
     ctx->step_window = (int32_t)W;
     return alloc_zero(ctx, &ctx->T.trig_mask, (size_t)ctx->n_slots);
@@ -1895,13 +1925,19 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
     std::vector<int32_t *> qs;
     if (ctx->queue_base)
         for (size_t b = 0; b < ctx->buckets.size(); b++) qs.push_back(ctx->queue_base + 2 * b);
+    LemsArgs la{ctx->d_lems_comps, ctx->n_lems_comps, ctx->d_lems_params, ctx->d_lems_pbegin, ctx->d_lems_state,
+                     ctx->n_slots, ctx->d_syn_ext, ctx->d_lems_peer, ctx->d_lems_flags, ctx->d_lems_poff,
+                     ctx->d_lems_tpos, ctx->d_lems_ttimes, ctx->d_pk_slot, ctx->d_pk_state, ctx->d_pk_isi,
+                     ctx->d_pk_window, ctx->d_pk_transient, ctx->d_pk_inst, ctx->d_pk_roff, ctx->d_inp_ext};
+    LemsCellArgs ca{ctx->d_acell_comps, ctx->d_acell_type, ctx->n_acells, ctx->d_acell_params,
+                                ctx->d_acell_pbegin, ctx->d_acell_vstate, ctx->d_acell_state, ctx->d_acell_poff};
     // the launches of steps [a0, a1), one range per launch
     auto issue = [&](int64_t a0, int64_t a1, bool pf) -> int {
         for (int64_t a = a0, b; a < a1; a = b) {
             // (initial steps send nothing and read no flags; one a launch in a network)
             b = std::min(a1, a + (per_step && a < 1 ? 1 : stride));
             const bool first = a == s0, last = b == s1;
-            if (ctx->n_grec > 0 && a >= 1) {
+            if (ctx->n_grec > 0 && a >= 1 && !ctx->lems_window_fn) {
                 // gate variables after step a - 1 into row a - 1, before step a changes them
                 // (one step per launch whenever gates are recorded)
                 const int64_t row = a - 1 - row0;
@@ -1912,12 +1948,17 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 HIPCHECK(ctx, hipGetLastError());
                 nl++;
             }
-            if (ctx->lems_fn && ctx->n_lems_comps > 0) {
+            if (ctx->lems_window_fn) {
+                int64_t aa = a, bb = b;
+                float dt = ctx->dt;
+                void *args[] = {&T, &la, &ca, &ctx->d_arec_begin, &ctx->d_arec_var, &ctx->d_arec_col, &aa, &bb, &row0, &dt};
+                HIPCHECK(ctx, hipModuleLaunchKernel(ctx->lems_window_fn,
+                                                    (unsigned)((ctx->n_acells + LEMS_SYN_COMPS - 1) / LEMS_SYN_COMPS), 1, 1,
+                                                    (unsigned)ctx->lems_threads, 1, 1, 0, ctx->stream, args, nullptr));
+                nl++;
+            }
+            if (ctx->lems_fn && ctx->n_lems_comps > 0 && !ctx->lems_window_fn) {
                 // generic synapses of step a: per-compartment currents for the kernels below
-                LemsArgs la{ctx->d_lems_comps, ctx->n_lems_comps, ctx->d_lems_params, ctx->d_lems_pbegin, ctx->d_lems_state,
-                     ctx->n_slots, ctx->d_syn_ext, ctx->d_lems_peer, ctx->d_lems_flags, ctx->d_lems_poff,
-                     ctx->d_lems_tpos, ctx->d_lems_ttimes, ctx->d_pk_slot, ctx->d_pk_state, ctx->d_pk_isi,
-                     ctx->d_pk_window, ctx->d_pk_transient, ctx->d_pk_inst, ctx->d_pk_roff, ctx->d_inp_ext};
                 int64_t st = a;
                 float dt = ctx->dt;
                 void *args[] = {&T, &la, &st, &dt};
@@ -1925,10 +1966,8 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                                                     1, 1, (unsigned)ctx->lems_threads, 1, 1, 0, ctx->stream, args, nullptr));
                 nl++;
             }
-            if (ctx->lems_cell_fn && ctx->n_acells > 0) {
+            if (ctx->lems_cell_fn && ctx->n_acells > 0 && !ctx->lems_window_fn) {
                 // point neurons of step a, after the synapse currents of the step
-                LemsCellArgs ca{ctx->d_acell_comps, ctx->d_acell_type, ctx->n_acells, ctx->d_acell_params,
-                                ctx->d_acell_pbegin, ctx->d_acell_vstate, ctx->d_acell_state, ctx->d_acell_poff};
                 int64_t st = a;
                 float dt = ctx->dt;
                 void *args[] = {&T, &ca, &st, &dt};
@@ -1999,7 +2038,7 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 if (pf) bk.launches++;
             }
             if (ctx->n_point > 0 && ctx->point_done) HIPCHECK(ctx, hipStreamWaitEvent(ctx->stream, ctx->point_done, 0));
-            if (T.trig_mask) {
+            if (T.trig_mask && ctx->n_slots > 0) {
                 hipLaunchKernelGGL(trig_fold_kernel, dim3((unsigned)((ctx->n_slots + 255) / 256)), dim3(256), 0, ctx->stream, T,
                                    ctx->n_slots, a, b, ctx->dt);
                 HIPCHECK(ctx, hipGetLastError());

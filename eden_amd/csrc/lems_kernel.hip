@@ -27,7 +27,9 @@
 // recipients and logged as a physical cell's is.
 //
 // The generated source (`lems_syn` and `lems_cell`) is inserted where
-// lems_synapse_functions.h is included.
+// lems_synapse_functions.h is included. It also defines EDENHIP_LEMS, for the kernels that the
+// model runs (compiling them is most of what creating a context costs): 0 neither synapses nor
+// point neurons, 1 synapses, 2 point neurons too, 3 both by lems_window_kernel.
 #define EDENHIP_LEMS_RATES 1
 #include "device_model.hpp"
 
@@ -50,9 +52,11 @@ __device__ __forceinline__ float lems_randof(float x, int seed, long long step, 
 
 #include "lems_synapse_functions.h"
 
-// One synapse instance's step: its current and conductance times the connection weight.
+// One synapse instance's step: its current and conductance times the connection weight. flags:
+// this step reads trigger flags (a later step of a launch has none, see trig_fold_kernel).
 __device__ __forceinline__ float2 lems_instance(const edenhip::DevTables &T, const edenhip::LemsArgs &L, int32_t g,
-                                                int32_t s, int32_t ty, float V, int64_t step, float t, float dt) {
+                                                int32_t s, int32_t ty, float V, int64_t step, float t, float dt,
+                                                bool flags) {
     using namespace edenhip;
     const bool init = step <= 0;
     int32_t *const trig_now = T.trig[(int)((step + 3) & 1)];
@@ -99,7 +103,7 @@ __device__ __forceinline__ float2 lems_instance(const edenhip::DevTables &T, con
         L.pk_state[k] = make_float2(tn, in);
     } else {
         bool flag = false;
-        if (!init) {
+        if (!init && flags) {
             flag = trig_now[s] != 0;
             if (flag) trig_now[s] = 0;
         }
@@ -129,32 +133,36 @@ __device__ __forceinline__ float2 lems_instance(const edenhip::DevTables &T, con
     return make_float2(i * weight, gx * weight);
 }
 
-// blockDim.x: LEMS_SYN_COMPS times the instances run side by side (at most LEMS_SYN_LANES)
-extern "C" __global__ void __launch_bounds__(edenhip::LEMS_SYN_COMPS * edenhip::LEMS_SYN_LANES)
-lems_syn_kernel(edenhip::DevTables T, edenhip::LemsArgs L, int64_t step, float dt) {
+// LDS of a workgroup of LEMS_SYN_COMPS compartments: two sets of their instances' values, so that
+// one may be summed while the next is filled, and their voltages.
+struct LemsShared {
+    float2 v[2][edenhip::LEMS_SYN_LANES][edenhip::LEMS_SYN_COMPS];
+    int32_t type[2][edenhip::LEMS_SYN_LANES][edenhip::LEMS_SYN_COMPS];
+    float V[edenhip::LEMS_SYN_COMPS];
+};
+
+// Totals of a compartment's synapses and LEMS inputs.
+struct LemsTotals {
+    float I_syn, G_syn, I_inp, G_inp;
+};
+
+// The synapses of a workgroup's compartments at a step (every lane calls it; blockDim.x:
+// LEMS_SYN_COMPS times the instances run side by side, at most LEMS_SYN_LANES). The first
+// LEMS_SYN_COMPS lanes get their compartment's totals.
+__device__ __forceinline__ LemsTotals lems_synapses(const edenhip::DevTables &T, const edenhip::LemsArgs &L,
+                                                    LemsShared &sh, int32_t g, int32_t base, int32_t cnt, int32_t most,
+                                                    float V, int64_t step, float t, float dt, bool flags) {
     using namespace edenhip;
     constexpr int C = LEMS_SYN_COMPS, INPUT = 1 << 30;
-    // two sets of values, so that one may be summed while the next is filled
-    __shared__ float2 s_v[2][LEMS_SYN_LANES][C];
-    __shared__ int32_t s_type[2][LEMS_SYN_LANES][C];
     const int c = threadIdx.x % C, lane = threadIdx.x / C, lanes = blockDim.x / C;
-    const int32_t idx = blockIdx.x * C + c;
-    const bool have = idx < L.n_comps;
-    const int32_t g = have ? L.comps[idx] : 0;
-    // time_f32 of the step, from the reference's double accumulation
-    const float t = (float)(step >= 1 ? T.t_row[step - 1] : 0.0);
-    const float V = T.V[g];
-    const int32_t base = T.syn_base[g], cnt = have ? T.syn_cnt[g] : 0;
-    int32_t most = cnt;        // of the workgroup's compartments
-    for (int m = 1; m < C; m <<= 1) most = max(most, __shfl_xor(most, m));
-    float I_syn = 0.0f, G_syn = 0.0f, I_agg = 0.0f, G_agg = 0.0f;
-    float I_inp = 0.0f, G_inp = 0.0f;   // LEMS inputs: i * weight per instance (eden/Eden.cpp:3929)
+    LemsTotals r{0.0f, 0.0f, 0.0f, 0.0f};   // I_inp: i * weight per instance (eden/Eden.cpp:3929)
+    float I_agg = 0.0f, G_agg = 0.0f;
     int32_t cur = -1;
     for (int32_t k0 = 0, set = 0; k0 < most; k0 += lanes, set ^= 1) {
         if (k0 + lane < cnt) {
             const int32_t s = base + 64 * (k0 + lane), ty = T.syn_type[s];
-            s_v[set][lane][c] = lems_instance(T, L, g, s, ty, V, step, t, dt);
-            s_type[set][lane][c] = ty | (L.flags && (L.flags[ty] & 1) ? INPUT : 0);
+            sh.v[set][lane][c] = lems_instance(T, L, g, s, ty, V, step, t, dt, flags);
+            sh.type[set][lane][c] = ty | (L.flags && (L.flags[ty] & 1) ? INPUT : 0);
         }
         __syncthreads();
         if (lane > 0) continue;
@@ -164,19 +172,19 @@ lems_syn_kernel(edenhip::DevTables T, edenhip::LemsArgs L, int64_t step, float d
             int32_t ty[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                v[j] = s_v[set][min(j0 + j, LEMS_SYN_LANES - 1)][c];
-                ty[j] = s_type[set][min(j0 + j, LEMS_SYN_LANES - 1)][c];
+                v[j] = sh.v[set][min(j0 + j, LEMS_SYN_LANES - 1)][c];
+                ty[j] = sh.type[set][min(j0 + j, LEMS_SYN_LANES - 1)][c];
             }
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 if (j0 + j >= n) continue;
                 if (ty[j] & INPUT) {
-                    I_inp += v[j].x;
-                    G_inp += v[j].y;
+                    r.I_inp += v[j].x;
+                    r.G_inp += v[j].y;
                     continue;
                 }
                 if (ty[j] != cur) {
-                    if (cur >= 0) { I_syn += I_agg; G_syn += G_agg; }
+                    if (cur >= 0) { r.I_syn += I_agg; r.G_syn += G_agg; }
                     I_agg = 0.0f; G_agg = 0.0f; cur = ty[j];
                 }
                 I_agg += v[j].x;
@@ -184,25 +192,46 @@ lems_syn_kernel(edenhip::DevTables T, edenhip::LemsArgs L, int64_t step, float d
             }
         }
     }
-    if (lane > 0 || !have) return;
-    I_syn += I_agg;
-    G_syn += G_agg;
-    L.syn_ext[g] = make_float2(I_syn, G_syn);
-    if (L.inp_ext) L.inp_ext[g] = make_float2(I_inp, G_inp);
+    r.I_syn += I_agg;
+    r.G_syn += G_agg;
+    return r;
 }
 
-extern "C" __global__ void __launch_bounds__(64)
-lems_cell_kernel(edenhip::DevTables T, edenhip::LemsCellArgs A, int64_t step, float dt) {
+// The largest of the first LEMS_SYN_COMPS lanes' values, the same ones in every group of lanes.
+__device__ __forceinline__ int32_t lems_most(int32_t x) {
+    for (int m = 1; m < edenhip::LEMS_SYN_COMPS; m <<= 1) x = max(x, __shfl_xor(x, m));
+    return x;
+}
+
+#if EDENHIP_LEMS == 1 || EDENHIP_LEMS == 2
+extern "C" __global__ void __launch_bounds__(edenhip::LEMS_SYN_COMPS * edenhip::LEMS_SYN_LANES)
+lems_syn_kernel(edenhip::DevTables T, edenhip::LemsArgs L, int64_t step, float dt) {
     using namespace edenhip;
-    const int32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= A.n) return;
-    const int32_t g = A.comps[idx], ty = A.type[idx];
-    const bool init = step <= 0;
+    __shared__ LemsShared sh;
+    const int c = threadIdx.x % LEMS_SYN_COMPS;
+    const int32_t idx = blockIdx.x * LEMS_SYN_COMPS + c;
+    const bool have = idx < L.n_comps;
+    const int32_t g = have ? L.comps[idx] : 0;
+    // time_f32 of the step, from the reference's double accumulation
     const float t = (float)(step >= 1 ? T.t_row[step - 1] : 0.0);
+    const int32_t cnt = have ? T.syn_cnt[g] : 0;
+    const LemsTotals r = lems_synapses(T, L, sh, g, T.syn_base[g], cnt, lems_most(cnt), T.V[g], step, t, dt, true);
+    if (threadIdx.x >= LEMS_SYN_COMPS || !have) return;
+    L.syn_ext[g] = make_float2(r.I_syn, r.G_syn);
+    if (L.inp_ext) L.inp_ext[g] = make_float2(r.I_inp, r.G_inp);
+}
+#endif
+
+#if EDENHIP_LEMS >= 2
+// A point neuron's step: synapse and input currents, the generated step, V (returned), its spike.
+__device__ __forceinline__ float lems_neuron(const edenhip::DevTables &T, const edenhip::LemsCellArgs &A, int32_t idx,
+                                             int32_t g, float V, int64_t step, float t, float dt, float I_syn,
+                                             bool has_inp, float I_inp, int at) {
+    using namespace edenhip;
+    const int32_t ty = A.type[idx];
+    const bool init = step <= 0;
     const int nxt = (int)((step + 3) & 1) ^ 1;
     // external current: synapses, then inputs (eden/Eden.cpp:6856-6880)
-    float I_syn = 0.0f;
-    if (T.syn_ext && T.syn_cnt[g] > 0) I_syn = T.syn_ext[g].x;
     float I_in = 0.0f;
     const int32_t pb = T.pulse_begin[g], pe = T.pulse_begin[g + 1];
     if (pe > pb) {
@@ -212,7 +241,7 @@ lems_cell_kernel(edenhip::DevTables T, edenhip::LemsCellArgs A, int64_t step, fl
         I_in += Ip;
         I_in += 0.0f;
     }
-    if (T.inp_ext && T.syn_cnt[g] > 0) I_in += T.inp_ext[g].x;   // LEMS inputs, after the native ones
+    if (has_inp) I_in += I_inp;   // LEMS inputs, after the native ones
     const float ext = I_syn + I_in;
     float *S = A.state + idx;
     int spike = 0;
@@ -220,12 +249,63 @@ lems_cell_kernel(edenhip::DevTables T, edenhip::LemsCellArgs A, int64_t step, fl
     lems_cell(ty, P, S, S, (long)A.n, t, dt, init ? 1 : 0, ext, (int)T.cell_seed[T.comp_cell[g]], (long long)step,
               &spike);
     const int32_t vs = A.v_state[ty];
-    if (vs >= 0) T.V[g] = S[(int64_t)vs * A.n];
+    if (vs >= 0) {
+        V = S[(int64_t)vs * A.n];
+        T.V[g] = V;
+    }
     if (spike) {
-        send_spike(T, g, nxt);
+        send_spike(T, g, nxt, at);
         log_event(T, T.ev_col[g], step);
     }
+    return V;
 }
+#endif
+
+#if EDENHIP_LEMS == 2
+extern "C" __global__ void __launch_bounds__(64)
+lems_cell_kernel(edenhip::DevTables T, edenhip::LemsCellArgs A, int64_t step, float dt) {
+    const int32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= A.n) return;
+    const int32_t g = A.comps[idx];
+    const float t = (float)(step >= 1 ? T.t_row[step - 1] : 0.0);
+    const bool has_syn = T.syn_cnt[g] > 0;
+    const float I_syn = T.syn_ext && has_syn ? T.syn_ext[g].x : 0.0f;
+    const bool has_inp = T.inp_ext && has_syn;
+    lems_neuron(T, A, idx, g, 0.0f, step, t, dt, I_syn, has_inp, has_inp ? T.inp_ext[g].x : 0.0f, 0);
+}
+#endif
+
+#if EDENHIP_LEMS == 3
+// Steps [s0, s1) of point neurons with their synapses and recorded state variables, in one launch:
+// where only they have generic synapses and none looks at another cell's voltage, nothing passes
+// between cells but spikes, whose delays span the window (trig_fold_kernel). Launches of the three
+// kernels for every step took 17.3 us a step with 700 cells of 30 synapses, this 6.6.
+extern "C" __global__ void __launch_bounds__(edenhip::LEMS_SYN_COMPS * edenhip::LEMS_SYN_LANES)
+lems_window_kernel(edenhip::DevTables T, edenhip::LemsArgs L, edenhip::LemsCellArgs A, const int32_t *rec_begin,
+                   const int32_t *rec_var, const int32_t *rec_col, int64_t s0, int64_t s1, int64_t row0, float dt) {
+    using namespace edenhip;
+    __shared__ LemsShared sh;
+    const int c = threadIdx.x % LEMS_SYN_COMPS;
+    const int32_t idx = blockIdx.x * LEMS_SYN_COMPS + c;
+    const bool have = idx < A.n, cell = have && threadIdx.x < LEMS_SYN_COMPS;
+    const int32_t g = have ? A.comps[idx] : 0;
+    const int32_t base = T.syn_base[g], cnt = have ? T.syn_cnt[g] : 0, most = lems_most(cnt);
+    int32_t rb = 0, re = 0;
+    if (cell && rec_begin) { rb = rec_begin[idx]; re = rec_begin[idx + 1]; }
+    if (threadIdx.x < LEMS_SYN_COMPS) sh.V[c] = T.V[g];
+    for (int64_t s = s0; s < s1; s++) {
+        __syncthreads();
+        const float t = (float)(s >= 1 ? T.t_row[s - 1] : 0.0), V = sh.V[c];
+        // state after the step before, before this one changes it
+        if (s >= 1)
+            for (int32_t r = rb; r < re; r++) trace_at(T, rec_col[r], s - 1 - row0) = A.state[(int64_t)rec_var[r] * A.n + idx];
+        const LemsTotals r = lems_synapses(T, L, sh, g, base, cnt, most, V, s, t, dt, s == s0);
+        if (cell)
+            sh.V[c] = lems_neuron(T, A, idx, g, V, s, t, dt, cnt > 0 ? r.I_syn : 0.0f, T.inp_ext && cnt > 0, r.I_inp,
+                                  (int)(s - s0));
+    }
+}
+#endif
 
 // Channels of the compartments run outside the compartment kernels, here with the user rate
 // ComponentTypes' generated lems_rate (gates of form RATE_LEMS); the statically compiled

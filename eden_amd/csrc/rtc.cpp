@@ -20,13 +20,14 @@ namespace {
 
 struct Compiled {
     hipModule_t module = nullptr;
-    hipFunction_t fn = nullptr, cell_fn = nullptr, ext_fn = nullptr;
+    hipFunction_t fn = nullptr, cell_fn = nullptr, ext_fn = nullptr, window_fn = nullptr;
 };
 
 }  // namespace
 
-int rtc_lems_kernel(const std::string &generated, hipFunction_t *fn, hipFunction_t *cell_fn, hipFunction_t *ext_fn,
-                    std::string &err) {
+int rtc_lems_kernel(const std::string &source, int kernels, hipFunction_t *fn, hipFunction_t *cell_fn, hipFunction_t *ext_fn,
+                    hipFunction_t *window_fn, std::string &err) {
+    const std::string generated = "#define EDENHIP_LEMS " + std::to_string(kernels) + "\n" + source;
     static std::mutex mu;
     static std::map<std::string, Compiled> cache;   // key: device arch + '\n' + source
     int dev = 0;
@@ -49,6 +50,7 @@ int rtc_lems_kernel(const std::string &generated, hipFunction_t *fn, hipFunction
         *fn = it->second.fn;
         *cell_fn = it->second.cell_fn;
         *ext_fn = it->second.ext_fn;
+        *window_fn = it->second.window_fn;
         return 0;
     }
     hiprtcProgram prog;
@@ -93,16 +95,18 @@ int rtc_lems_kernel(const std::string &generated, hipFunction_t *fn, hipFunction
         err = "hipModuleLoadData of the synapse kernel failed";
         return -1;
     }
-    if (hipModuleGetFunction(&c.fn, c.module, "lems_syn_kernel") != hipSuccess ||
-        hipModuleGetFunction(&c.cell_fn, c.module, "lems_cell_kernel") != hipSuccess ||
-        hipModuleGetFunction(&c.ext_fn, c.module, "ext_channels_kernel_rtc") != hipSuccess) {
-        err = "lems_syn_kernel / lems_cell_kernel / ext_channels_kernel_rtc not found in the compiled module";
+    auto missing = [&](hipFunction_t *f, const char *name) { return hipModuleGetFunction(f, c.module, name) != hipSuccess; };
+    if (((kernels == 1 || kernels == 2) && missing(&c.fn, "lems_syn_kernel")) ||
+        (kernels == 2 && missing(&c.cell_fn, "lems_cell_kernel")) ||
+        (kernels == 3 && missing(&c.window_fn, "lems_window_kernel")) || missing(&c.ext_fn, "ext_channels_kernel_rtc")) {
+        err = "a kernel of lems_kernel.hip is not in the compiled module";
         return -1;
     }
     cache[key] = c;
     *fn = c.fn;
     *cell_fn = c.cell_fn;
     *ext_fn = c.ext_fn;
+    *window_fn = c.window_fn;
     return 0;
 }
 
