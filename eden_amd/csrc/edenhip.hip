@@ -1532,9 +1532,9 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         b.lds = (size_t)tree_lds(b.nmax, b.nvmax, b.ngmax, b.nctmax, b.ninmax, b.words_max, b.cxmax_lds, ctx->n_gates,
                                  ctx->n_stypes, b.split).total *
                 sizeof(float);
-        // lean_tree_kernel runs a bucket of lean cells: also where its blocks, twice the LDS, leave
-        // fewer cells in flight (481 rows of 4,096 cells of up to 400 compartments 5.3 -> 4.3 ms, of
-        // up to 2,000 11.5 -> 10.9 ms)
+        // lean_tree_kernel runs every bucket of lean cells, also where its blocks, twice the LDS,
+        // leave fewer cells in flight (481 rows of 4,096 cells of up to 400 compartments 5.3 -> 3.4
+        // ms, of up to 2,000 11.5 -> 8.4; with tree_kernel for the 512-thread bucket alone 9.0)
         b.lean = b.lean && !ctx->tree_net;
         if (b.lean) b.lds = (size_t)b.lean_bytes;
         const int nt = b.tpb + (b.split ? 64 : 0);
