@@ -916,6 +916,16 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     // Hines schedules of the tree cells, planned in parallel (independent per cell); cells
     // with malformed parents are left unplanned here and rejected in the loop below
     std::vector<WavePlan> plans(d->n_cells);
+    // size limits: in a network a lane takes one or two compartments instead of up to four, since
+    // its compartments' synapses take their trips to memory one after another (limits 256 / 512 /
+    // 1024 -> 64 / 128 / 512, 400 steps: 48 trees of 20 to 150 compartments 5.2 -> 4.3 ms, 1,024 of
+    // them 6.5 -> 5.3, 48 of 100 to 600 7.1 -> 5.4, 256 active ones of 60 to 250 10.3 -> 7.2;
+    // without synapses more lanes are slower, 256 active trees of 60 to 160 14.5 -> 21 ms)
+    int32_t limits[4];
+    std::copy(ctx->opt.size_limits, ctx->opt.size_limits + 4, limits);
+    if (d->comp_spike_begin[NC] > 0 && limits[0] == 0 && limits[1] == 0 && limits[2] == 0 && limits[3] == 0) {
+        limits[0] = 64; limits[1] = 128; limits[2] = 512; limits[3] = MAX_TREE_N;
+    }
     {
         auto plan_one = [&](int c) {
             const int64_t c0 = d->cell_comp_begin[c];
@@ -923,7 +933,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
             if (n <= 1 || n > MAX_TREE_N || d->parent[c0] != -1) return;
             for (int32_t i = 1; i < n; i++)
                 if (d->parent[c0 + i] < 0 || d->parent[c0 + i] >= i) return;
-            const int32_t tpb = choose_tpb(n, ctx->opt.threads_per_cell, ctx->opt.size_limits);
+            const int32_t tpb = choose_tpb(n, ctx->opt.threads_per_cell, limits);
             // wave 0 updates the root compartment during the first Hines phase; 2- and 4-wave
             // cells also update their gates on the last cable wave (they have no channel wave)
             const bool gates_on_last = tpb == 128 || tpb == 256;
@@ -955,7 +965,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
             continue;
         }
         if (n > MAX_TREE_N) return fail(ctx, EDENHIP_E_LIMIT, "cell with more than 2047 compartments");
-        const int32_t tpb = choose_tpb(n, ctx->opt.threads_per_cell, ctx->opt.size_limits);
+        const int32_t tpb = choose_tpb(n, ctx->opt.threads_per_cell, limits);
         const WavePlan &P = plans[c];
         TreeCell tc{};
         tc.gate_off = (int64_t)gqv.size();

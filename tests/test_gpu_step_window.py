@@ -2,7 +2,7 @@
 (lems_window_kernel), several steps per launch (trig_fold_kernel): traces,
 spikes, synaptic deliveries, last voltages and saved states equal the oracle's and those of
 launches of one step, over delays around the shortest that allow a window and the longest window,
-spikes that find one pending, odd chunks, forced window lengths, captured graphs, and float times
+spikes that find one pending, odd chunks, other workgroup sizes, forced window lengths, captured graphs, and float times
 whose step windows overlap (launches of one step)."""
 import dataclasses
 
@@ -32,7 +32,7 @@ def _run(m, **opt):
     ((0.05, 0.1), 25.0, {}), ((0.1, 0.2), 25.0, {}), ((0.1, 30.0), 25.0, dict(chunk_steps=37)),
     ((1.0, 4.0), 25.0, {}), ((1.0, 4.0), 25.0, dict(network_window=5, chunk_steps=101)),
     ((1.0, 4.0), 25.0, dict(use_graph=True, chunk_steps=300)), ((1.7, 20.0), 25.0, dict(chunk_steps=1)),
-    ((3.0, 12.0), 25.0, {}), ((1.0, 4.0), 23.7, {}), ((1.0, 4.0), 12.5, {})])
+    ((3.0, 12.0), 25.0, {}), ((1.0, 4.0), 25.0, dict(size_limits=(256, 512, 1024, 2047))), ((1.0, 4.0), 23.7, {}), ((1.0, 4.0), 12.5, {})])
 def test_windows_equal_oracle_and_single_steps(delay_ms, dt, opt):
     m = _model(delay_ms, 21, dt)
     tr, ev, syn, v, blob = _run(m, **opt)
