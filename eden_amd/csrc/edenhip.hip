@@ -24,6 +24,7 @@
 
 #include "../../include/edenhip.h"
 #include "device_model.hpp"
+#include "event_order.hpp"
 #include "kernels.hpp"
 #include "rtc.hpp"
 #include "tree_schedule.hpp"
@@ -2355,24 +2356,7 @@ int edenhip_read_events(edenhip_ctx *ctx, int64_t *col, int64_t *row, int64_t ma
         HIPCHECK(ctx, hipMemcpyAsync(ev.data(), ctx->T.events, cnt * sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
         HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
     }
-    // by (row, column): counted into rows, then the few events of each row sorted (many events),
-    // or sorted outright (few)
-    if ((int64_t)cnt * 4 > ctx->total_rows) {
-        std::vector<uint32_t> at((size_t)ctx->total_rows + 2, 0u);
-        for (int64_t x : ev) at[(size_t)(x >> 24) + 1]++;
-        for (size_t r = 1; r < at.size(); r++) at[r] += at[r - 1];
-        std::vector<int64_t> by_row(cnt);
-        for (int64_t x : ev) by_row[at[(size_t)(x >> 24)]++] = x;
-        ev.swap(by_row);
-        for (size_t b = 0; b < ev.size();) {
-            size_t e = b + 1;
-            while (e < ev.size() && (ev[e] >> 24) == (ev[b] >> 24)) e++;
-            std::sort(ev.begin() + (int64_t)b, ev.begin() + (int64_t)e);
-            b = e;
-        }
-    } else {
-        std::sort(ev.begin(), ev.end());
-    }
+    order_events(ev, ctx->total_rows);
     int64_t k = 0;
     for (int64_t x : ev) {
         const int64_t r = x >> 24, c = x & 0xFFFFFF;
