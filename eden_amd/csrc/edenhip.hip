@@ -82,7 +82,10 @@ struct Bucket {
     bool split = false;   // one extra wave runs the channel phase concurrently
     bool lean = true;     // lean_tree_kernel runs it: every cell is TreeCell::lean
     int64_t lean_bytes = 0;   // its largest cell's LDS there
-    const void *kernel(bool net) const { return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(tpb, split, net); }
+    bool gates_lds = true;    // the general kernel's gate table is in LDS, else in global memory
+    const void *kernel(bool net) const {
+        return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(tpb, split, net, gates_lds);
+    }
     std::vector<int32_t> order;    // tree-cell indices, largest first
     int32_t nmax = 0;
     int32_t nvmax = 0;        // voltage slots in LDS (1 for a constant tree, else its size)
@@ -1538,21 +1541,31 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         const int cw = ctx->opt.channel_wave[b.tpb == 64 ? 0 : b.tpb == 128 ? 1 : b.tpb == 256 ? 2 : 3];
         const bool rule = b.tpb == 512 || (b.tpb == 64 && (int64_t)bc.size() <= 4 * (int64_t)ctx->n_cu);
         b.split = (cw > 0 || (cw == 0 && rule)) && ctx->opt.persistent >= 0 && !ctx->tree_net;
-        // complex-compartment records go to LDS when they take at most 20 KiB
-        b.cxmax_lds = b.cxmax <= 256 ? b.cxmax : 0;
-        b.lds = (size_t)tree_lds(b.nmax, b.nvmax, b.ngmax, b.nctmax, b.ninmax, b.words_max, b.cxmax_lds, ctx->n_gates,
-                                 ctx->n_stypes, b.split).total *
-                sizeof(float);
         // lean_tree_kernel runs every bucket of lean cells, also where its blocks, twice the LDS,
         // leave fewer cells in flight (481 rows of 4,096 cells of up to 400 compartments 5.3 -> 3.4
         // ms, of up to 2,000 11.5 -> 8.4; with tree_kernel for the 512-thread bucket alone 9.0)
         b.lean = b.lean && !ctx->tree_net;
-        if (b.lean) b.lds = (size_t)b.lean_bytes;
         const int nt = b.tpb + (b.split ? 64 : 0);
-        const void *kp = b.kernel(ctx->tree_net);
-        if (!kp) return fail(ctx, EDENHIP_E_LIMIT, "no tree kernel for the chosen workgroup size");
         int per_cu = 0;
-        HIPCHECK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, nt, b.lds));
+        if (b.lean) {
+            b.lds = (size_t)b.lean_bytes;
+            HIPCHECK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, b.kernel(false), nt, b.lds));
+        } else {
+            // complex-compartment records go to LDS when they take at most 24 KiB. Where a cell's
+            // tables do not fit with them and the gate table, first the gate table stays in global
+            // memory (small, and in cache), then the records, then both
+            const int32_t cx = b.cxmax <= 256 ? b.cxmax : 0;
+            for (int drop = 0; drop < 4 && per_cu <= 0; drop++) {
+                b.gates_lds = (drop & 1) == 0;
+                b.cxmax_lds = (drop & 2) == 0 ? cx : 0;
+                b.lds = (size_t)tree_lds(b.nmax, b.nvmax, b.ngmax, b.nctmax, b.ninmax, b.words_max, b.cxmax_lds,
+                                         b.gates_lds ? ctx->n_gates : 0, ctx->n_stypes, b.split).total *
+                        sizeof(float);
+                const void *kp = b.kernel(ctx->tree_net);
+                if (!kp && b.gates_lds) return fail(ctx, EDENHIP_E_LIMIT, "no tree kernel for the chosen workgroup size");
+                if (kp) HIPCHECK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, nt, b.lds));
+            }
+        }
         if (per_cu <= 0) return fail(ctx, EDENHIP_E_LIMIT, "tree kernel does not fit on a CU (LDS)");
         b.grid = (int)std::min<int64_t>((int64_t)bc.size(), (int64_t)per_cu * ctx->n_cu);
         TRY(upload(ctx, &b.d_cells, bc));

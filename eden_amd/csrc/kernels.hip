@@ -240,8 +240,12 @@ __device__ __forceinline__ void channel_phase(const DGate *gates, const uint32_t
 // the point kernel does, and a compartment with spike recipients sends its spikes to the
 // next step's flags; both are complex compartments, so the per-slot code of the other
 // compartments is unchanged and the NET = false kernels carry none of it.
-template <int TPB, bool SPLIT, bool NET>
-__global__ void __launch_bounds__(TPB + (SPLIT ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(4)))
+// FORM: the cable group's threads; one more where the gate table, up to 16 KiB, is read from global
+// memory. That is for the largest cells, whose other tables leave no room for it: a binary tree with
+// HH channels on every compartment, in a model of 64 channel types, takes up to 1,743 compartments
+// with the table in LDS and 1,937 without.
+template <int FORM, bool SPLIT, bool NET>
+__global__ void __launch_bounds__((FORM & ~1) + (SPLIT ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(4)))
 tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const DSynType *__restrict__ stypes_g,
             int n_stypes, const TreeCell *__restrict__ cells, const int32_t *__restrict__ task_order, int32_t n_tasks,
             int32_t *__restrict__ queue, const uint32_t *__restrict__ words_g, const int32_t *__restrict__ pos_g,
@@ -250,14 +254,17 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
             const uint32_t *__restrict__ cflag_g, const TreeComplex *__restrict__ cx_g, int32_t cxmax_lds, int32_t nmax,
             int32_t nvmax, int32_t ngmax, int32_t nctmax, int32_t ninmax, int32_t words_max, int64_t s0, int64_t s1,
             int64_t row0, float dt) {
+    constexpr int TPB = FORM & ~1;
+    constexpr bool GATES_LDS = (FORM & 1) == 0;
     constexpr int K = TREE_SLOTS;
     constexpr int NT = TPB + (SPLIT ? 64 : 0);
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int32_t s_task;
     // dynamic LDS, laid out by tree_lds()
-    const TreeLds L = tree_lds(nmax, nvmax, ngmax, nctmax, ninmax, words_max, cxmax_lds, n_gates, n_stypes, SPLIT);
+    const TreeLds L =
+        tree_lds(nmax, nvmax, ngmax, nctmax, ninmax, words_max, cxmax_lds, GATES_LDS ? n_gates : 0, n_stypes, SPLIT);
     float *sm = reinterpret_cast<float *>(smem);
-    DGate *gates = reinterpret_cast<DGate *>(sm + L.gtab);
+    const DGate *const gates = GATES_LDS ? reinterpret_cast<const DGate *>(sm + L.gtab) : gates_g;
     DSynType *stypes = reinterpret_cast<DSynType *>(sm + L.stab);
     TreeComplex *sCX = reinterpret_cast<TreeComplex *>(sm + L.cx);
     // Hines node records, 16 bytes at position p: sDX(p) = (diagonal, rhs), then sU(p) =
@@ -275,7 +282,8 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
     uint32_t *sW = reinterpret_cast<uint32_t *>(sm + L.w);   // schedule block: round headers, task words
     const int tid = threadIdx.x;
     const bool cable = !SPLIT || tid < TPB;
-    for (int i = tid; i < n_gates; i += NT) gates[i] = gates_g[i];
+    if constexpr (GATES_LDS)
+        for (int i = tid; i < n_gates; i += NT) reinterpret_cast<DGate *>(sm + L.gtab)[i] = gates_g[i];
     for (int i = tid; i < n_stypes; i += NT) stypes[i] = stypes_g[i];
 
     for (;;) {
@@ -1179,13 +1187,16 @@ lean_tree_kernel(DevTables T, const DGate *__restrict__ gates_g, const TreeCell 
     }
 }
 
+// (a cell of up to 512 compartments leaves room for the gate table at any channel count)
 template <bool SPLIT, bool NET>
-static const void *tree_kernel_of(int tpb) {
-    switch (tpb) {
+static const void *tree_kernel_of(int form) {
+    switch (form) {
     case 64: return reinterpret_cast<const void *>(&tree_kernel<64, SPLIT, NET>);
     case 128: return reinterpret_cast<const void *>(&tree_kernel<128, SPLIT, NET>);
     case 256: return reinterpret_cast<const void *>(&tree_kernel<256, SPLIT, NET>);
     case 512: return reinterpret_cast<const void *>(&tree_kernel<512, SPLIT, NET>);
+    case 257: return reinterpret_cast<const void *>(&tree_kernel<257, SPLIT, NET>);
+    case 513: return reinterpret_cast<const void *>(&tree_kernel<513, SPLIT, NET>);
     default: return nullptr;
     }
 }
@@ -1201,9 +1212,10 @@ static const void *lean_kernel_of(int tpb) {
     }
 }
 
-const void *tree_kernel_ptr(int tpb, bool split, bool net) {
-    if (net) return split ? nullptr : tree_kernel_of<false, true>(tpb);
-    return split ? tree_kernel_of<true, false>(tpb) : tree_kernel_of<false, false>(tpb);
+const void *tree_kernel_ptr(int tpb, bool split, bool net, bool gates_lds) {
+    const int form = tpb + (gates_lds ? 0 : 1);
+    if (net) return split ? nullptr : tree_kernel_of<false, true>(form);
+    return split ? tree_kernel_of<true, false>(form) : tree_kernel_of<false, false>(form);
 }
 
 const void *lean_tree_kernel_ptr(int tpb, bool split) {

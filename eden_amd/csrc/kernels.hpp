@@ -52,7 +52,8 @@ constexpr int TREE_SLOTS = 4;        // compartments per thread
 // ((diagonal, rhs), (Ui, Uj)) | sIn [nmax] float2
 // (only with Poisson inputs) | sV [nbuf][nvmax+1] | sQ [ngmax] | sGT [ngmax] | sF [nbuf][nctmax]
 // | sCT [nctmax] | sIL [ninmax] | schedule block [words_max] (16-byte aligned) | sCX [cxmax]
-// TreeComplex (only when the records are staged in LDS) | gate table [n_gates] DGate |
+// TreeComplex (only when the records are staged in LDS) | gate table [n_gates] DGate (n_gates 0
+// where it is read from global memory) |
 // synapse types [n_stypes] DSynType; nbuf = 2 when a separate wave runs the channel phase,
 // else 1. nvmax: voltage slots of the bucket's cells (1 for a constant tree, whose only
 // voltage read from LDS is the root's, else its compartment count).
@@ -133,8 +134,9 @@ constexpr int NET_QUAD_GROUPS[] = {1, 2, 4, 6, 8, 10, 12, 16};
 constexpr int NET_QUAD_MAX = 16;
 
 // net: the variant for networks (synapses on tree compartments, spikes sent to recipients),
-// launched one step at a time; only without a channel wave.
-const void *tree_kernel_ptr(int tpb, bool split, bool net = false);
+// launched one step at a time; only without a channel wave. gates_lds: the gate table is in LDS,
+// else read from global memory (256 and 512 threads only). Null where there is none.
+const void *tree_kernel_ptr(int tpb, bool split, bool net, bool gates_lds = true);
 // for buckets whose cells are all TreeCell::lean
 const void *lean_tree_kernel_ptr(int tpb, bool split);
 // Dynamic LDS of lean_tree_kernel: a few scalars, from LEAN_X on the right-hand sides (two more
