@@ -130,7 +130,7 @@ struct edenhip_ctx {
     int32_t *d_grec_col = nullptr;
     int64_t *d_grec_src = nullptr;
     int32_t n_grec = 0;
-    bool grec_other = false;      // some are not point neurons' state variables
+    bool steps_overlap = false;   // two float step windows [t, t + dt) of the run overlap
     std::vector<std::vector<int64_t>> ev_expand;   // dev event column -> desc columns
     int64_t chunk_rows = 0, last_row0 = 0, last_rows = 0;
     DevTables T{};
@@ -298,7 +298,8 @@ static std::vector<double> row_times(float dt, double t_final) {
     return ts;
 }
 
-static int build_step_window(edenhip_ctx *ctx, const edenhip_model_desc *d);
+static int32_t step_window_len(const edenhip_ctx *ctx, const edenhip_model_desc *d);
+static int build_step_window(edenhip_ctx *ctx, int32_t W);
 static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std::vector<int32_t> &point,
                         const std::vector<DSynType> &stypes);
 
@@ -880,7 +881,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     }
     ctx->n_dev_cols += (int32_t)grec.size();
     // state read back between launches: recorded gate variables need one launch per step
-    // (but for point neurons' state variables, which lems_window_kernel records: build_step_window)
+    // (but for point neurons' state variables, which lems_window_kernel records)
     ctx->window_opt = ctx->opt.persistent < 0 ? -1 : ctx->opt.network_window;
     if (!grec.empty()) {
         ctx->opt.persistent = -1;
@@ -898,6 +899,10 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     // time table
     std::vector<double> ts = row_times(d->dt, d->t_final);
     ctx->total_rows = (int64_t)ts.size();
+    for (size_t j = 0; j < ts.size(); j++) {
+        const double next = j + 1 < ts.size() ? ts[j + 1] : ts[j] + (double)d->dt;
+        if ((float)ts[j] + d->dt > (float)next) ctx->steps_overlap = true;
+    }
 
     // cells: point (1 compartment) vs tree
     std::vector<int32_t> point;
@@ -920,15 +925,37 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     // Hines schedules of the tree cells, planned in parallel (independent per cell); cells
     // with malformed parents are left unplanned here and rejected in the loop below
     std::vector<WavePlan> plans(d->n_cells);
-    // size limits: in a network a lane takes one or two compartments instead of up to four, since
-    // its compartments' synapses take their trips to memory one after another (limits 256 / 512 /
-    // 1024 -> 64 / 128 / 512, 400 steps: 48 trees of 20 to 150 compartments 5.2 -> 4.3 ms, 1,024 of
-    // them 6.5 -> 5.3, 48 of 100 to 600 7.1 -> 5.4, 256 active ones of 60 to 250 10.3 -> 7.2;
-    // without synapses more lanes are slower, 256 active trees of 60 to 160 14.5 -> 21 ms)
+    // Steps per launch of the general network path (trig_fold_kernel). Generic synapses and point
+    // neurons that lems_window_kernel does not take (it takes models where only point neurons have
+    // generic synapses, and none a peer), channel pre-passes and other recorded state have kernels
+    // of their own between the steps, and keep launches of one.
+    bool windows = x_comp.empty();
+    if (ctx->n_acells > 0) {
+        for (const auto &r : grec) windows = windows && acell_slot[r.first] >= 0;
+        for (int64_t g = 0; g < NC && windows && lems; g++)
+            windows = d->comp_syn_begin[g + 1] == d->comp_syn_begin[g] || acell_slot[g] >= 0;
+        if (lems && d->abi_version >= 3 && LS->peer)
+            for (int64_t k = 0; k < n_syn && windows; k++) windows = LS->peer[k] < 0;
+    } else {
+        windows = windows && d->comp_spike_begin[NC] > 0 && !lems && grec.empty();
+    }
+    const int32_t window_len = windows ? step_window_len(ctx, d) : 1;
+    // size limits: in a network that runs windows a lane takes one or two compartments instead of
+    // up to four, since its compartments' synapses take their trips to memory one after another
+    // (limits 256 / 512 / 1024 -> 64 / 128 / 512, 201 steps: 4 trees of 20 to 150 compartments 2.4 ->
+    // 1.9 ms, 48 of 100 to 600 3.3 -> 2.7, 256 active ones of 60 to 250 4.9 -> 3.8, 1,024 of 20 to 150
+    // 3.1 -> 2.8; slower only for 600 of 700 to 1,500, 4.1 -> 5.4; without synapses more lanes are
+    // slower, 256 active trees of 60 to 160 14.5 -> 21 ms). With launches of one step every size in
+    // use is a launch of its own, forked and joined in each step, so the limits leave few sizes
+    // (256 / 512 / 1024, 64 / 128 / 512 and 256 / 512 / 512: 48 trees of 20 to 150 compartments 7.9,
+    // 13.5 and 7.9 ms, 100 of 700 to 1,900 13.9, 11.1 and 11.1, 48 with generic synapses 8.2, 11.2
+    // and 8.2)
     int32_t limits[4];
     std::copy(ctx->opt.size_limits, ctx->opt.size_limits + 4, limits);
     if (d->comp_spike_begin[NC] > 0 && limits[0] == 0 && limits[1] == 0 && limits[2] == 0 && limits[3] == 0) {
-        limits[0] = 64; limits[1] = 128; limits[2] = 512; limits[3] = MAX_TREE_N;
+        limits[0] = window_len > 1 ? 64 : 256;
+        limits[1] = window_len > 1 ? 128 : 512;
+        limits[2] = 512; limits[3] = MAX_TREE_N;
     }
     {
         auto plan_one = [&](int c) {
@@ -1217,7 +1244,6 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         std::vector<int32_t> begin((size_t)ctx->n_acells + 1, 0), var, col;
         for (const auto &r : grec)
             if (acell_slot[r.first] >= 0) begin[(size_t)acell_slot[r.first] + 1]++;
-            else ctx->grec_other = true;
         for (size_t i = 1; i < begin.size(); i++) begin[i] += begin[i - 1];
         var.resize((size_t)begin.back());
         col.resize(var.size());
@@ -1378,11 +1404,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         gen += "\n";
         gen += rates_src ? std::string(rates_src)
                          : std::string("__device__ float lems_rate(int, float) { return 0.0f; }\n");
-        // lems_window_kernel: only point neurons have generic synapses, none a peer
-        bool window = ctx->n_acells > 0 && !ctx->grec_other;
-        for (int64_t g = 0; g < NC && window && lems; g++) window = syn_cnt[g] == 0 || acell_slot[g] >= 0;
-        for (int64_t k = 0; k < n_syn && window && lems && d->abi_version >= 3 && LS->peer; k++) window = LS->peer[k] < 0;
-        if (window) TRY(build_step_window(ctx, d));
+        if (ctx->n_acells > 0) TRY(build_step_window(ctx, window_len));
         const int kernels = ctx->step_window > 1 ? 3 : ctx->n_acells > 0 ? 2 : lems && n_syn > 0 ? 1 : 0;
         std::string err;
         hipFunction_t syn_fn = nullptr, cell_fn = nullptr, ext_fn = nullptr, window_fn = nullptr;
@@ -1593,7 +1615,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     }
     HIPCHECK(ctx, hipEventCreateWithFlags(&ctx->ev_start, hipEventDisableTiming));
     TRY(build_netwin(ctx, d, point, st));
-    if (!ctx->netwin && !lems && ctx->n_acells == 0 && ctx->n_grec == 0) TRY(build_step_window(ctx, d));
+    if (!ctx->netwin && ctx->n_acells == 0) TRY(build_step_window(ctx, window_len));
     TRY(upload(ctx, &ctx->d_snaps, ctx->snaps));
     for (const auto &sn : ctx->snaps) ctx->snap_max = std::max(ctx->snap_max, (int64_t)sn.bytes);
     if (!ctx->desc_to_dev_col.empty()) {
@@ -1608,29 +1630,21 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     return 0;
 }
 
-// Whether two float step windows [t, t + dt) of the model overlap.
-static bool step_windows_overlap(const edenhip_model_desc *d) {
-    const std::vector<double> ts = row_times(d->dt, d->t_final);
-    for (size_t j = 0; j < ts.size(); j++) {
-        const double next = j + 1 < ts.size() ? ts[j + 1] : ts[j] + (double)d->dt;
-        if ((float)ts[j] + d->dt > (float)next) return true;
-    }
-    return false;
-}
-
-// The general network path: how many steps a launch may run (trig_fold_kernel). Generic synapses
-// and point neurons that lems_window_kernel does not take, channel pre-passes and other recorded
-// state have kernels of their own between the steps, and keep launches of one.
-static int build_step_window(edenhip_ctx *ctx, const edenhip_model_desc *d) {
+// How many steps a launch of the general network path may run: every spike's delay covers them.
+static int32_t step_window_len(const edenhip_ctx *ctx, const edenhip_model_desc *d) {
     const int32_t nw = ctx->window_opt;
-    if (!ctx->network || nw < 0 || ctx->n_xcomp > 0 || step_windows_overlap(d)) return 0;
+    if (nw < 0 || ctx->steps_overlap) return 1;
     double dmin = INFINITY;
     for (int64_t k = 0; k < d->comp_spike_begin[d->n_comps]; k++)
         dmin = std::min(dmin, (double)d->syn_delay[d->spike_target[k]]);
     const double most = std::min(64.0, std::floor(dmin / (double)d->dt) - 2.0);
     const int64_t W = nw > 0 ? std::min<int64_t>(nw, (int64_t)most) : (int64_t)most;
+    return (int32_t)std::max<int64_t>(W, 1);
+}
+
+static int build_step_window(edenhip_ctx *ctx, int32_t W) {
     if (W < 2) return 0;
-    ctx->step_window = (int32_t)W;
+    ctx->step_window = W;
     return alloc_zero(ctx, &ctx->T.trig_mask, (size_t)ctx->n_slots);
 }
 
@@ -1779,7 +1793,7 @@ static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std
     // The one case a window cannot decide, a pending arrival that lies in two consecutive step
     // windows [t, t + dt), needs windows that overlap. Where the float times do not, as with any
     // dt of whole microseconds, no window has to be checked against step order.
-    ctx->net_free = !step_windows_overlap(d) && ctx->opt.network_window != -2;
+    ctx->net_free = !ctx->steps_overlap && ctx->opt.network_window != -2;
     ctx->net_W = W;
     ctx->net_cur = 0;
     ctx->netwin = true;

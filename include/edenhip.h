@@ -331,8 +331,9 @@ typedef struct edenhip_options {
                                      where delays allow it, else one */
     int32_t size_limits[4];       /* largest tree cell (compartments) given 64, 128, 256 and
                                      512 threads; all 0 = 256, 512, 1024, 2047, or in a
-                                     network 64, 128, 512, 2047. A cell takes
-                                     the first size whose limit holds it (each limit at most 4
+                                     network of tree cells 64, 128, 512, 2047 where launches run
+                                     several steps and 256, 512, 512, 2047 where they run one.
+                                     A cell takes the first size whose limit holds it (each limit at most 4
                                      compartments per thread; the 512 limit must be 2047).
                                      eden_amd.autotune picks them by timing short runs. */
     int32_t channel_wave[4];      /* (abi_version >= 3) tree cells with 64, 128, 256, 512 threads:
