@@ -1602,8 +1602,14 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
             HIPCHECK(ctx, hipEventCreate(&b.p1));
         }
     }
+    // point cells beside the tree buckets, on a stream of their own; with launches of one step and
+    // several buckets on the main one, before its bucket, as a fourth stream to fork and join in
+    // every step costs more than it hides (201 steps with 20 point cells: 48 trees of 100 to 600
+    // compartments, three buckets, 13.6 -> 12.0 ms; 100 of 700 to 1,900, two, 13.9 -> 12.6; one
+    // bucket of 1,024 trees 14.6 beside it, 15.0 before it)
     ctx->point_stream = ctx->stream;
-    if (ctx->n_point > 0 && !ctx->buckets.empty() && ctx->buckets.size() < 4) {
+    const bool single = (ctx->network || ctx->opt.persistent < 0) && window_len == 1;
+    if (ctx->n_point > 0 && !ctx->buckets.empty() && ctx->buckets.size() < (single ? 2u : 4u)) {
         TRY(pool_stream(ctx, (int)ctx->buckets.size(), &ctx->point_stream));
         HIPCHECK(ctx, hipEventCreateWithFlags(&ctx->point_done, hipEventDisableTiming));
     }
