@@ -745,7 +745,7 @@ __device__ __forceinline__ void exptwo_step(const DSynType &st, float V, float &
 // expTwo dynamics, per-type aggregation in list order (eden/Eden.cpp:3636-3740). The fields
 // of SYN_CHUNK synapses are loaded before any of them is computed (independent loads in
 // flight); the accumulation stays sequential in synapse order.
-// A point cell has many, a tree's compartment mostly one or two: 8 and 2 at a time.
+// A point cell has many, a tree's compartment mostly one or two: 8 and 2 (or 8, SYN_MANY) at a time.
 template <int SYN_CHUNK>
 __device__ __forceinline__ void synapses_step(const DevTables &T, const DSynType *__restrict__ stypes, int32_t base,
                                               int32_t cnt, float V, bool init, float t, float dt, int now,

@@ -83,8 +83,10 @@ struct Bucket {
     bool lean = true;     // lean_tree_kernel runs it: every cell is TreeCell::lean
     int64_t lean_bytes = 0;   // its largest cell's LDS there
     bool gates_lds = true;    // the general kernel's gate table is in LDS, else in global memory
+    bool long_lists = false;  // a compartment with SYN_MANY synapses or more
     const void *kernel(bool net) const {
-        return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(tpb, split, net, gates_lds);
+        const int form = tpb + (gates_lds ? 0 : 1) + (net && long_lists ? 2 : 0);
+        return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(form, split, net);
     }
     std::vector<int32_t> order;    // tree-cell indices, largest first
     int32_t nmax = 0;
@@ -1535,6 +1537,8 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         b->nctmax = std::max(b->nctmax, cells[i].n_ctask);
         b->words_max = std::max(b->words_max, cells[i].words_len);
         b->cxmax = std::max(b->cxmax, cells[i].n_cx);
+        for (int64_t g = cells[i].comp_begin; g < cells[i].comp_begin + cells[i].n && !lems; g++)
+            b->long_lists = b->long_lists || syn_cnt[(size_t)g] >= SYN_MANY;
         b->lean = b->lean && cells[i].lean != 0;
         b->lean_bytes = std::max(b->lean_bytes, lean_lds(cells[i].lean_len, cells[i].n));
     }

@@ -240,12 +240,13 @@ __device__ __forceinline__ void channel_phase(const DGate *gates, const uint32_t
 // the point kernel does, and a compartment with spike recipients sends its spikes to the
 // next step's flags; both are complex compartments, so the per-slot code of the other
 // compartments is unchanged and the NET = false kernels carry none of it.
-// FORM: the cable group's threads; one more where the gate table, up to 16 KiB, is read from global
-// memory. That is for the largest cells, whose other tables leave no room for it: a binary tree with
+// FORM: the cable group's threads; two more where a compartment's synapses are read eight at a time
+// (a bucket with a long list, SYN_MANY), else two; one more where the gate table, up to 16 KiB, is
+// read from global memory. That is for the largest cells, whose other tables leave no room for it: a binary tree with
 // HH channels on every compartment, in a model of 64 channel types, takes up to 1,743 compartments
 // with the table in LDS and 1,937 without.
 template <int FORM, bool SPLIT, bool NET>
-__global__ void __launch_bounds__((FORM & ~1) + (SPLIT ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__((FORM & ~3) + (SPLIT ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(4)))
 tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const DSynType *__restrict__ stypes_g,
             int n_stypes, const TreeCell *__restrict__ cells, const int32_t *__restrict__ task_order, int32_t n_tasks,
             int32_t *__restrict__ queue, const uint32_t *__restrict__ words_g, const int32_t *__restrict__ pos_g,
@@ -254,7 +255,7 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
             const uint32_t *__restrict__ cflag_g, const TreeComplex *__restrict__ cx_g, int32_t cxmax_lds, int32_t nmax,
             int32_t nvmax, int32_t ngmax, int32_t nctmax, int32_t ninmax, int32_t words_max, int64_t s0, int64_t s1,
             int64_t row0, float dt) {
-    constexpr int TPB = FORM & ~1;
+    constexpr int TPB = FORM & ~3;
     constexpr bool GATES_LDS = (FORM & 1) == 0;
     constexpr int K = TREE_SLOTS;
     constexpr int NT = TPB + (SPLIT ? 64 : 0);
@@ -541,8 +542,8 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
                             G_in += e2.y;
                         }
                     } else {
-                        synapses_step<2>(T, stypes, cx.syn_base, cx.syn_cnt, V[j], init, t, dt, (int)((s + 3) & 1), s,
-                                         I_syn, G_syn);
+                        synapses_step<(FORM & 2) ? 8 : 2>(T, stypes, cx.syn_base, cx.syn_cnt, V[j], init, t, dt,
+                                                          (int)((s + 3) & 1), s, I_syn, G_syn);
                     }
                 }
             }
@@ -1197,8 +1198,18 @@ static const void *tree_kernel_of(int form) {
     case 512: return reinterpret_cast<const void *>(&tree_kernel<512, SPLIT, NET>);
     case 257: return reinterpret_cast<const void *>(&tree_kernel<257, SPLIT, NET>);
     case 513: return reinterpret_cast<const void *>(&tree_kernel<513, SPLIT, NET>);
-    default: return nullptr;
     }
+    if constexpr (NET) {
+        switch (form) {
+        case 66: return reinterpret_cast<const void *>(&tree_kernel<66, SPLIT, NET>);
+        case 130: return reinterpret_cast<const void *>(&tree_kernel<130, SPLIT, NET>);
+        case 258: return reinterpret_cast<const void *>(&tree_kernel<258, SPLIT, NET>);
+        case 514: return reinterpret_cast<const void *>(&tree_kernel<514, SPLIT, NET>);
+        case 259: return reinterpret_cast<const void *>(&tree_kernel<259, SPLIT, NET>);
+        case 515: return reinterpret_cast<const void *>(&tree_kernel<515, SPLIT, NET>);
+        }
+    }
+    return nullptr;
 }
 
 template <bool SPLIT>
@@ -1212,8 +1223,7 @@ static const void *lean_kernel_of(int tpb) {
     }
 }
 
-const void *tree_kernel_ptr(int tpb, bool split, bool net, bool gates_lds) {
-    const int form = tpb + (gates_lds ? 0 : 1);
+const void *tree_kernel_ptr(int form, bool split, bool net) {
     if (net) return split ? nullptr : tree_kernel_of<false, true>(form);
     return split ? tree_kernel_of<true, false>(form) : tree_kernel_of<false, false>(form);
 }

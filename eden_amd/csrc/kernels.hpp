@@ -133,10 +133,16 @@ struct NetClasses {
 constexpr int NET_QUAD_GROUPS[] = {1, 2, 4, 6, 8, 10, 12, 16};
 constexpr int NET_QUAD_MAX = 16;
 
-// net: the variant for networks (synapses on tree compartments, spikes sent to recipients),
-// launched one step at a time; only without a channel wave. gates_lds: the gate table is in LDS,
-// else read from global memory (256 and 512 threads only). Null where there is none.
-const void *tree_kernel_ptr(int tpb, bool split, bool net, bool gates_lds = true);
+// form: a workgroup's threads without a channel wave (64, 128, 256, 512), plus 1 where the gate
+// table is read from global memory (256 and 512 only), plus 2 in a network where a compartment's
+// synapses are read eight at a time. net: the variant for networks (synapses on tree compartments,
+// spikes sent to recipients), only without a channel wave. Null where there is none.
+const void *tree_kernel_ptr(int form, bool split, bool net);
+// Synapses of one compartment from which a bucket's kernel reads eight at a time, each a register
+// set of its own: 48 trees of 20 to 150 compartments with 50 on each soma 11.9 -> 11.4 ms, 120 24.2 ->
+// 22.1, 600 trees with 50 7.5 -> 6.7 (401 and 201 steps). Below, two at a time: most have one or two,
+// and the same trees with 470 synapses in all take 2.3 ms, with eight at a time 2.6.
+constexpr int SYN_MANY = 16;
 // for buckets whose cells are all TreeCell::lean
 const void *lean_tree_kernel_ptr(int tpb, bool split);
 // Dynamic LDS of lean_tree_kernel: a few scalars, from LEAN_X on the right-hand sides (two more
