@@ -116,6 +116,8 @@ struct DevTables {
 
 // lems_syn_kernel's workgroup: compartments, and at most so many instances of each at a time.
 constexpr int LEMS_SYN_COMPS = 16, LEMS_SYN_LANES = 32;
+// its dynamic LDS in bytes: voltages, then 24 bytes a thread (LemsLane)
+constexpr unsigned lems_syn_lds(unsigned threads, bool wave_comps) { return 256u + (wave_comps ? 0u : 24u * threads); }
 
 // Arguments of lems_syn_kernel (the generic LEMS synapse kernel, compiled at run time from
 // lems_kernel.hip): shared by that compilation and the host code that launches it.
@@ -140,6 +142,7 @@ struct LemsArgs {
     const int32_t *pk_inst;       // per spiker: randof instance
     const int32_t *pk_roff;       // per spiker: randof invocation offset
     float2 *inp_ext;              // [NC] per-compartment (I, G) of the LEMS inputs of the step, or null
+    int32_t wave_comps;           // 1: 64 compartments a workgroup, one lane each
 };
 
 // Arguments of lems_cell_kernel (LEMS point neurons, compiled at run time with the synapse

@@ -204,6 +204,11 @@ struct edenhip_ctx {
     // generic LEMS synapses: the run-time compiled synapse kernel and its tables
     hipFunction_t lems_fn = nullptr;
     int32_t lems_threads = 64;    // of a workgroup of lems_syn_kernel
+    bool lems_wave = true;        // 64 compartments, a lane each
+    unsigned lems_blocks(int32_t comps) const {
+        const int32_t each = lems_wave ? 64 : LEMS_SYN_COMPS;
+        return (unsigned)((comps + each - 1) / each);
+    }
     int32_t *d_lems_comps = nullptr;
     int32_t n_lems_comps = 0;
     float *d_lems_params = nullptr, *d_lems_state = nullptr;
@@ -1317,6 +1322,10 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         for (int32_t g : lc) most = std::max(most, syn_cnt[g]);
         while (lanes < most && lanes < LEMS_SYN_LANES) lanes *= 2;
         ctx->lems_threads = LEMS_SYN_COMPS * lanes;
+        // a lane a compartment where it has one instance, or two and the compartments alone fill the
+        // chip's waves (eight a SIMD): four lanes each would be idle by half
+        ctx->lems_wave = most <= 1 || (most == 2 && lc.size() > (size_t)LEMS_SYN_COMPS * 8 * 4 * ctx->n_cu);
+        if (ctx->lems_wave) ctx->lems_threads = 64;
         int32_t smax = 1;
         for (int t = 0; t < LS->n_types; t++) smax = std::max(smax, LS->n_state[t]);
         const int64_t np = lems_param_count(LS->param_begin, LS->n_types, d->abi_version >= 4 ? LS->n_params : 0);
@@ -1976,9 +1985,10 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
     LemsArgs la{ctx->d_lems_comps, ctx->n_lems_comps, ctx->d_lems_params, ctx->d_lems_pbegin, ctx->d_lems_state,
                      ctx->n_slots, ctx->d_syn_ext, ctx->d_lems_peer, ctx->d_lems_flags, ctx->d_lems_poff,
                      ctx->d_lems_tpos, ctx->d_lems_ttimes, ctx->d_pk_slot, ctx->d_pk_state, ctx->d_pk_isi,
-                     ctx->d_pk_window, ctx->d_pk_transient, ctx->d_pk_inst, ctx->d_pk_roff, ctx->d_inp_ext};
+                     ctx->d_pk_window, ctx->d_pk_transient, ctx->d_pk_inst, ctx->d_pk_roff, ctx->d_inp_ext, ctx->lems_wave ? 1 : 0};
     LemsCellArgs ca{ctx->d_acell_comps, ctx->d_acell_type, ctx->n_acells, ctx->d_acell_params,
                                 ctx->d_acell_pbegin, ctx->d_acell_vstate, ctx->d_acell_state, ctx->d_acell_poff};
+    const unsigned lems_lds = lems_syn_lds((unsigned)ctx->lems_threads, ctx->lems_wave);
     // the launches of steps [a0, a1), one range per launch
     auto issue = [&](int64_t a0, int64_t a1, bool pf) -> int {
         for (int64_t a = a0, b; a < a1; a = b) {
@@ -2000,9 +2010,8 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 int64_t aa = a, bb = b;
                 float dt = ctx->dt;
                 void *args[] = {&T, &la, &ca, &ctx->d_arec_begin, &ctx->d_arec_var, &ctx->d_arec_col, &aa, &bb, &row0, &dt};
-                HIPCHECK(ctx, hipModuleLaunchKernel(ctx->lems_window_fn,
-                                                    (unsigned)((ctx->n_acells + LEMS_SYN_COMPS - 1) / LEMS_SYN_COMPS), 1, 1,
-                                                    (unsigned)ctx->lems_threads, 1, 1, 0, ctx->stream, args, nullptr));
+                HIPCHECK(ctx, hipModuleLaunchKernel(ctx->lems_window_fn, ctx->lems_blocks(ctx->n_acells), 1, 1,
+                                                    (unsigned)ctx->lems_threads, 1, 1, lems_lds, ctx->stream, args, nullptr));
                 nl++;
             }
             if (ctx->lems_fn && ctx->n_lems_comps > 0 && !ctx->lems_window_fn) {
@@ -2010,8 +2019,8 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 int64_t st = a;
                 float dt = ctx->dt;
                 void *args[] = {&T, &la, &st, &dt};
-                HIPCHECK(ctx, hipModuleLaunchKernel(ctx->lems_fn, (unsigned)((ctx->n_lems_comps + LEMS_SYN_COMPS - 1) / LEMS_SYN_COMPS),
-                                                    1, 1, (unsigned)ctx->lems_threads, 1, 1, 0, ctx->stream, args, nullptr));
+                HIPCHECK(ctx, hipModuleLaunchKernel(ctx->lems_fn, ctx->lems_blocks(ctx->n_lems_comps), 1, 1,
+                                                    (unsigned)ctx->lems_threads, 1, 1, lems_lds, ctx->stream, args, nullptr));
                 nl++;
             }
             if (ctx->lems_cell_fn && ctx->n_acells > 0 && !ctx->lems_window_fn) {

@@ -14,8 +14,8 @@
 // place (the generated code reads an instance's whole present state before writing).
 //
 // An instance is a chain of dependent loads and divisions, so its latency, not its work, is what
-// a step costs: the instances of a compartment go to lanes of their own, LEMS_SYN_COMPS
-// compartments side by side (their slots are neighbours: 64-byte accesses) times as many
+// a step costs: the instances of a compartment (where it has several) go to lanes of their own,
+// LEMS_SYN_COMPS compartments side by side (their slots are neighbours: 64-byte accesses) times as many
 // instances as the workgroup has room for, and leave their currents in LDS; one lane per
 // compartment then sums them in list order. 700 cells with 30 synapses each: 49.9 us a step with
 // a lane per compartment, now 9.5 us.
@@ -133,63 +133,80 @@ __device__ __forceinline__ float2 lems_instance(const edenhip::DevTables &T, con
     return make_float2(i * weight, gx * weight);
 }
 
-// LDS of a workgroup of LEMS_SYN_COMPS compartments: two sets of their instances' values, so that
-// one may be summed while the next is filled, and their voltages.
-struct LemsShared {
-    float2 v[2][edenhip::LEMS_SYN_LANES][edenhip::LEMS_SYN_COMPS];
-    int32_t type[2][edenhip::LEMS_SYN_LANES][edenhip::LEMS_SYN_COMPS];
-    float V[edenhip::LEMS_SYN_COMPS];
+// A workgroup: LEMS_SYN_COMPS compartments with as many lanes each as instances run side by side
+// (at most LEMS_SYN_LANES), or, where a compartment has one instance (or many compartments two), a
+// wave of 64 compartments (L.wave_comps). Its LDS (lems_syn_lds bytes, dynamic): the compartments' voltages,
+// then per lane of a compartment two sets of its instances' values, so that one may be summed
+// while the next is filled. 12 KiB for the most lanes there can be would leave only 13 workgroups a
+// CU in flight, where large populations have more. 100,000 cells with a synapse each 21.1 -> 14.2 us a
+// step (17.5 with a lane a compartment and no LDS), 200,000 with two 40.0 -> 24.5, 50,000 point
+// neurons with two 7.0 -> 5.1.
+struct LemsLane {
+    float2 v[2][edenhip::LEMS_SYN_COMPS];
+    int32_t type[2][edenhip::LEMS_SYN_COMPS];
 };
+extern __shared__ __align__(16) float lems_shared[];
+__device__ __forceinline__ LemsLane *lems_lanes() { return reinterpret_cast<LemsLane *>(lems_shared + 64); }
 
 // Totals of a compartment's synapses and LEMS inputs.
 struct LemsTotals {
     float I_syn, G_syn, I_inp, G_inp;
 };
 
-// The synapses of a workgroup's compartments at a step (every lane calls it; blockDim.x:
-// LEMS_SYN_COMPS times the instances run side by side, at most LEMS_SYN_LANES). The first
-// LEMS_SYN_COMPS lanes get their compartment's totals.
+// The synapses of a workgroup's compartments at a step (every lane calls it; c: the lane's
+// compartment, lane: its place among the compartment's lanes). The compartments' first lanes get
+// their totals.
 __device__ __forceinline__ LemsTotals lems_synapses(const edenhip::DevTables &T, const edenhip::LemsArgs &L,
-                                                    LemsShared &sh, int32_t g, int32_t base, int32_t cnt, int32_t most,
-                                                    float V, int64_t step, float t, float dt, bool flags) {
+                                                    int c, int lane, int32_t g, int32_t base, int32_t cnt,
+                                                    int32_t most, float V, int64_t step, float t, float dt, bool flags) {
     using namespace edenhip;
-    constexpr int C = LEMS_SYN_COMPS, INPUT = 1 << 30;
-    const int c = threadIdx.x % C, lane = threadIdx.x / C, lanes = blockDim.x / C;
+    constexpr int INPUT = 1 << 30;
+    const int lanes = L.wave_comps ? 1 : blockDim.x / LEMS_SYN_COMPS;
+    LemsLane *const sh = lems_lanes();
     LemsTotals r{0.0f, 0.0f, 0.0f, 0.0f};   // I_inp: i * weight per instance (eden/Eden.cpp:3929)
     float I_agg = 0.0f, G_agg = 0.0f;
     int32_t cur = -1;
+    auto add = [&](float2 v, int32_t ty) {
+        if (ty & INPUT) {
+            r.I_inp += v.x;
+            r.G_inp += v.y;
+            return;
+        }
+        if (ty != cur) {
+            if (cur >= 0) { r.I_syn += I_agg; r.G_syn += G_agg; }
+            I_agg = 0.0f; G_agg = 0.0f; cur = ty;
+        }
+        I_agg += v.x;
+        G_agg += v.y;
+    };
     for (int32_t k0 = 0, set = 0; k0 < most; k0 += lanes, set ^= 1) {
         if (k0 + lane < cnt) {
             const int32_t s = base + 64 * (k0 + lane), ty = T.syn_type[s];
-            sh.v[set][lane][c] = lems_instance(T, L, g, s, ty, V, step, t, dt, flags);
-            sh.type[set][lane][c] = ty | (L.flags && (L.flags[ty] & 1) ? INPUT : 0);
+            const float2 v = lems_instance(T, L, g, s, ty, V, step, t, dt, flags);
+            const int32_t kind = ty | (L.flags && (L.flags[ty] & 1) ? INPUT : 0);
+            if (lanes == 1) {
+                add(v, kind);
+            } else {
+                sh[lane].v[set][c] = v;
+                sh[lane].type[set][c] = kind;
+            }
         }
+        if (lanes == 1) continue;
         __syncthreads();
         if (lane > 0) continue;
+        // (lanes is a multiple of 4)
         const int n = min(cnt - k0, lanes);
         for (int j0 = 0; j0 < n; j0 += 4) {
             float2 v[4];
             int32_t ty[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                v[j] = sh.v[set][min(j0 + j, LEMS_SYN_LANES - 1)][c];
-                ty[j] = sh.type[set][min(j0 + j, LEMS_SYN_LANES - 1)][c];
+                v[j] = sh[j0 + j].v[set][c];
+                ty[j] = sh[j0 + j].type[set][c];
             }
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (j0 + j >= n) continue;
-                if (ty[j] & INPUT) {
-                    r.I_inp += v[j].x;
-                    r.G_inp += v[j].y;
-                    continue;
-                }
-                if (ty[j] != cur) {
-                    if (cur >= 0) { r.I_syn += I_agg; r.G_syn += G_agg; }
-                    I_agg = 0.0f; G_agg = 0.0f; cur = ty[j];
-                }
-                I_agg += v[j].x;
-                G_agg += v[j].y;
-            }
+            for (int j = 0; j < 4; j++)
+                if (j0 + j < n) add(v[j], ty[j]);
         }
     }
     r.I_syn += I_agg;
@@ -197,26 +214,35 @@ __device__ __forceinline__ LemsTotals lems_synapses(const edenhip::DevTables &T,
     return r;
 }
 
-// The largest of the first LEMS_SYN_COMPS lanes' values, the same ones in every group of lanes.
+// The largest value of a workgroup's compartments (a wave holds all of them, or several times).
 __device__ __forceinline__ int32_t lems_most(int32_t x) {
-    for (int m = 1; m < edenhip::LEMS_SYN_COMPS; m <<= 1) x = max(x, __shfl_xor(x, m));
+    for (int m = 1; m < 64; m <<= 1) x = max(x, __shfl_xor(x, m));
     return x;
 }
+
+// Compartments of a workgroup, and a lane's compartment and place there.
+struct LemsPlace {
+    int comps, c, lane;
+    __device__ __forceinline__ explicit LemsPlace(const edenhip::LemsArgs &L) {
+        comps = L.wave_comps ? 64 : edenhip::LEMS_SYN_COMPS;
+        c = threadIdx.x & (comps - 1);
+        lane = L.wave_comps ? 0 : threadIdx.x / edenhip::LEMS_SYN_COMPS;
+    }
+};
 
 #if EDENHIP_LEMS == 1 || EDENHIP_LEMS == 2
 extern "C" __global__ void __launch_bounds__(edenhip::LEMS_SYN_COMPS * edenhip::LEMS_SYN_LANES)
 lems_syn_kernel(edenhip::DevTables T, edenhip::LemsArgs L, int64_t step, float dt) {
     using namespace edenhip;
-    __shared__ LemsShared sh;
-    const int c = threadIdx.x % LEMS_SYN_COMPS;
-    const int32_t idx = blockIdx.x * LEMS_SYN_COMPS + c;
+    const LemsPlace at(L);
+    const int32_t idx = blockIdx.x * at.comps + at.c;
     const bool have = idx < L.n_comps;
     const int32_t g = have ? L.comps[idx] : 0;
     // time_f32 of the step, from the reference's double accumulation
     const float t = (float)(step >= 1 ? T.t_row[step - 1] : 0.0);
     const int32_t cnt = have ? T.syn_cnt[g] : 0;
-    const LemsTotals r = lems_synapses(T, L, sh, g, T.syn_base[g], cnt, lems_most(cnt), T.V[g], step, t, dt, true);
-    if (threadIdx.x >= LEMS_SYN_COMPS || !have) return;
+    const LemsTotals r = lems_synapses(T, L, at.c, at.lane, g, T.syn_base[g], cnt, lems_most(cnt), T.V[g], step, t, dt, true);
+    if (at.lane > 0 || !have) return;
     L.syn_ext[g] = make_float2(r.I_syn, r.G_syn);
     if (L.inp_ext) L.inp_ext[g] = make_float2(r.I_inp, r.G_inp);
 }
@@ -284,24 +310,25 @@ extern "C" __global__ void __launch_bounds__(edenhip::LEMS_SYN_COMPS * edenhip::
 lems_window_kernel(edenhip::DevTables T, edenhip::LemsArgs L, edenhip::LemsCellArgs A, const int32_t *rec_begin,
                    const int32_t *rec_var, const int32_t *rec_col, int64_t s0, int64_t s1, int64_t row0, float dt) {
     using namespace edenhip;
-    __shared__ LemsShared sh;
-    const int c = threadIdx.x % LEMS_SYN_COMPS;
-    const int32_t idx = blockIdx.x * LEMS_SYN_COMPS + c;
-    const bool have = idx < A.n, cell = have && threadIdx.x < LEMS_SYN_COMPS;
+    const LemsPlace at(L);
+    const int c = at.c;
+    const int32_t idx = blockIdx.x * at.comps + c;
+    const bool have = idx < A.n, cell = have && at.lane == 0;
+    float *const sV = lems_shared;
     const int32_t g = have ? A.comps[idx] : 0;
     const int32_t base = T.syn_base[g], cnt = have ? T.syn_cnt[g] : 0, most = lems_most(cnt);
     int32_t rb = 0, re = 0;
     if (cell && rec_begin) { rb = rec_begin[idx]; re = rec_begin[idx + 1]; }
-    if (threadIdx.x < LEMS_SYN_COMPS) sh.V[c] = T.V[g];
+    if (at.lane == 0) sV[c] = T.V[g];
     for (int64_t s = s0; s < s1; s++) {
         __syncthreads();
-        const float t = (float)(s >= 1 ? T.t_row[s - 1] : 0.0), V = sh.V[c];
+        const float t = (float)(s >= 1 ? T.t_row[s - 1] : 0.0), V = sV[c];
         // state after the step before, before this one changes it
         if (s >= 1)
             for (int32_t r = rb; r < re; r++) trace_at(T, rec_col[r], s - 1 - row0) = A.state[(int64_t)rec_var[r] * A.n + idx];
-        const LemsTotals r = lems_synapses(T, L, sh, g, base, cnt, most, V, s, t, dt, s == s0);
+        const LemsTotals r = lems_synapses(T, L, c, at.lane, g, base, cnt, most, V, s, t, dt, s == s0);
         if (cell)
-            sh.V[c] = lems_neuron(T, A, idx, g, V, s, t, dt, cnt > 0 ? r.I_syn : 0.0f, T.inp_ext && cnt > 0, r.I_inp,
+            sV[c] = lems_neuron(T, A, idx, g, V, s, t, dt, cnt > 0 ? r.I_syn : 0.0f, T.inp_ext && cnt > 0, r.I_inp,
                                   (int)(s - s0));
     }
 }
