@@ -6,9 +6,9 @@ Each candidate is a full context (its own Hines schedules) advanced `steps` step
 the whole run), timed from the host around `edenhip_run` after one warm-up run; the state is
 rewound between runs. Short runs are cheaper but their timings need not carry over to the
 whole run, where the buckets' tails overlap differently. The
-search is coordinate-wise over the three movable limits, from the size rule (256, 512, 1024):
-a limit moves down when the larger workgroup is faster for the cells between the two values
-by more than `margin` (default 2 %: whole runs of one context vary by about 1 % from run to
+search is coordinate-wise over the three movable limits, from the library's size rule: 256,
+512, 1024, and in a network the smaller limits that Simulation.size_limits() reports. A limit
+moves when another value is faster by more than `margin` (default 2 %: whole runs of one context vary by about 1 % from run to
 run, so a smaller gain is not told apart from noise and the present limits are kept).
 
     from eden_amd.autotune import autotune, autotune_channel_wave
@@ -25,11 +25,15 @@ import copy
 import sys
 import time
 
+import numpy as np
+
 from .model import Simulation
 
 DEFAULT = (256, 512, 1024, 2047)
 # candidate values per movable limit (each at most 4 compartments per thread)
 CANDIDATES = ((128, 192, 256), (384, 448, 512), (768, 896, 1024))
+# the same in a network, whose own limits are 64, 128, 512 or 256, 512, 512
+NETWORK_CANDIDATES = ((64, 128, 256), (128, 256, 512), (512, 768, 1024))
 
 
 def _shortened(model, steps):
@@ -65,6 +69,16 @@ def time_limits(model, limits, steps=None, repeats=2, device=0, channel_wave=Non
     return best
 
 
+def size_rule(model, device=0):
+    """(limits, candidates): the library's own size limits for the model, and the values to try
+    for each. A network's limits depend on how many steps a launch may run, so a context is
+    asked for them."""
+    if model.comp_spike_begin is None or np.asarray(model.comp_spike_begin)[-1] == 0:
+        return DEFAULT, CANDIDATES
+    with Simulation(model, device=device) as sim:
+        return sim.size_limits(), NETWORK_CANDIDATES
+
+
 def autotune(model, steps=None, repeats=2, device=0, verbose=False, margin=0.02):
     """Returns (limits, report): the fastest size limits found and every timing taken."""
     if model.n_comps == model.n_cells:
@@ -79,9 +93,10 @@ def autotune(model, steps=None, repeats=2, device=0, verbose=False, margin=0.02)
             print(f"[autotune] limits {tuple(limits)}: {t * 1e3:.2f} ms / {what}", file=sys.stderr, flush=True)
         return t
 
-    best = list(DEFAULT)
+    rule, candidates = size_rule(model, device)
+    best = list(rule)
     best_t = measure(best)
-    for k, cands in enumerate(CANDIDATES):
+    for k, cands in enumerate(candidates):
         for v in cands:
             if v == best[k]:
                 continue

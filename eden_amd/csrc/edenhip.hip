@@ -161,6 +161,7 @@ struct edenhip_ctx {
         int64_t launches;
     };
     std::vector<GraphEntry> graphs;
+    int32_t limits[4] = {};       // size limits in force
     int32_t window_opt = 0;       // options.network_window as given, -1 with launches of one step
     int32_t step_window = 1;      // steps per launch of the general network path (trig_fold_kernel)
     int n_cu = 256;
@@ -957,12 +958,14 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     // (256 / 512 / 1024, 64 / 128 / 512 and 256 / 512 / 512: 48 trees of 20 to 150 compartments 7.9,
     // 13.5 and 7.9 ms, 100 of 700 to 1,900 13.9, 11.1 and 11.1, 48 with generic synapses 8.2, 11.2
     // and 8.2)
-    int32_t limits[4];
+    int32_t *const limits = ctx->limits;
     std::copy(ctx->opt.size_limits, ctx->opt.size_limits + 4, limits);
-    if (d->comp_spike_begin[NC] > 0 && limits[0] == 0 && limits[1] == 0 && limits[2] == 0 && limits[3] == 0) {
-        limits[0] = window_len > 1 ? 64 : 256;
-        limits[1] = window_len > 1 ? 128 : 512;
-        limits[2] = 512; limits[3] = MAX_TREE_N;
+    if (limits[0] == 0 && limits[1] == 0 && limits[2] == 0 && limits[3] == 0) {
+        const bool net = d->comp_spike_begin[NC] > 0;
+        limits[0] = net && window_len > 1 ? 64 : 256;
+        limits[1] = net && window_len > 1 ? 128 : 512;
+        limits[2] = net ? 512 : 1024;
+        limits[3] = MAX_TREE_N;
     }
     {
         auto plan_one = [&](int c) {
@@ -2515,6 +2518,12 @@ int edenhip_network_stats(edenhip_ctx *ctx, int32_t *window_steps, int64_t *wind
         if (ctx->netwin) HIPCHECK(ctx, hipMemcpy(&n, ctx->N.n_deliv, sizeof(n), hipMemcpyDeviceToHost));
         *synaptic_events = ctx->netwin ? (int64_t)n : -1;
     }
+    return 0;
+}
+
+int edenhip_size_limits(const edenhip_ctx *ctx, int32_t limits[4]) {
+    if (!ctx || !limits) return EDENHIP_E_INVALID;
+    std::copy(ctx->limits, ctx->limits + 4, limits);
     return 0;
 }
 

@@ -486,6 +486,12 @@ class Simulation:
                     "network_stats")
         return w.value, n.value, r.value, e.value
 
+    def size_limits(self):
+        """Size limits in force: the option's, or those the library chose for the model."""
+        limits = (C.c_int32 * 4)()
+        self._check(self.lib.edenhip_size_limits(self.h, limits), "size_limits")
+        return tuple(limits)
+
     def launch_shape(self):
         t, k = C.c_int32(), C.c_int32()
         self._check(self.lib.edenhip_launch_shape(self.h, C.byref(t), C.byref(k)), "launch_shape")

@@ -448,6 +448,9 @@ int edenhip_get_kernel_cells(const edenhip_ctx *ctx, int32_t i, int32_t *cells, 
 int edenhip_network_stats(edenhip_ctx *ctx, int32_t *window_steps, int64_t *windows, int64_t *windows_rerun,
                           int64_t *synaptic_events);
 
+/* The size limits in force: edenhip_options.size_limits, or those chosen where all are 0. */
+int edenhip_size_limits(const edenhip_ctx *ctx, int32_t limits[4]);
+
 /* Describe the launch shape chosen for the tree-cell kernel (autotuned or given). */
 int edenhip_launch_shape(const edenhip_ctx *ctx, int32_t *threads_per_cell, int32_t *slots_per_thread);
 

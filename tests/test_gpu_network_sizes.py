@@ -6,7 +6,7 @@ import dataclasses
 import numpy as np
 import pytest
 
-from eden_amd import configs, lems
+from eden_amd import autotune, configs, lems
 from eden_amd.model import Simulation
 from oracle import oracle
 
@@ -41,3 +41,15 @@ def test_sizes_follow_the_steps_per_launch(delay_ms, generic, opt, limits):
     assert len(er) > 0
     assert np.array_equal(tr, ref) and np.array_equal(v, rv)
     assert np.array_equal(ev[0], ec) and np.array_equal(ev[1], er)
+
+
+def test_autotuner_starts_from_the_networks_limits():
+    m = configs.mixed_network(tree_sizes=SIZES, n_point=6, n_conn=150, t_final_ms=5.0, seed=8)
+    assert autotune.size_rule(m) == (WINDOW, autotune.NETWORK_CANDIDATES)
+    limits, report = autotune.autotune(m, steps=60, repeats=1)
+    print(f"[autotune] {limits} from {report}", flush=True)
+    times = dict(report)
+    assert report[0][0] == WINDOW and times[limits] <= times[WINDOW]
+    with Simulation(m) as a, Simulation(m, size_limits=limits) as b:
+        assert a.size_limits() == WINDOW and b.size_limits() == limits
+        assert np.array_equal(a.run_all(), b.run_all())
