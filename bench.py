@@ -378,10 +378,10 @@ def main():
         one_step(psim)
         infos = psim.kernel_infos()
         for ki in infos:
-            acc = kern.setdefault(ki["name"], dict(ki, total_ms=0.0, launches=0))
+            acc = kern.setdefault(ki["symbol"], dict(ki, total_ms=0.0, launches=0))
             acc["total_ms"] += ki["total_ms"]
             acc["launches"] += ki["launches"]
-        msg = ", ".join(f"{ki['name']} {ki['total_ms']:.2f} ms/{ki['launches']} (grid {ki['grid']}, "
+        msg = ", ".join(f"{ki['symbol']} {ki['total_ms']:.2f} ms/{ki['launches']} (grid {ki['grid']}, "
                         f"LDS {ki['lds_bytes']} B)" for ki in infos)
         print(f"[bench] profiled run: {msg}", file=sys.stderr, flush=True)
     net = None
@@ -415,13 +415,13 @@ def main():
         wkey += ")"
     traffic = None
     for f in sorted(glob.glob(os.path.join(ROOT, "profiles", "*_traffic.md"))):
-        traffic = traffic or read_traffic(f, dom["name"], wkey)
-    lds = lds_entry(dom["name"], wkey)
+        traffic = traffic or read_traffic(f, dom["symbol"], wkey)
+    lds = lds_entry(dom["symbol"], wkey)
     roofline = dict(bound="hbm", achieved=achieved / 1e9, peak=HBM_PEAK / 1e9, unit="GB/s",
-                    frac=achieved / HBM_PEAK, traffic=traffic, kernel=dom["name"],
+                    frac=achieved / HBM_PEAK, traffic=traffic, kernel=dom["symbol"],
                     kernel_cells=int(dom["cells"]), kernel_comps=int(dom["comps"]),
                     bytes_per_launch=bytes_per_launch, launch_ms=per_launch_ms,
-                    all_kernels={k["name"]: dict(ms_per_launch=k["total_ms"] / max(1, k["launches"]),
+                    all_kernels={k["symbol"]: dict(ms_per_launch=k["total_ms"] / max(1, k["launches"]),
                                                  cells=int(k["cells"]), comps=int(k["comps"]))
                                  for k in kern.values()},
                     # every kernel of the run together: algorithmic bytes of the whole workload

@@ -117,6 +117,7 @@ EXPORTS = {
     "edenhip_kernel_stats": (C.c_int, [C.c_void_p, C.POINTER(C.c_double), C.POINTER(C.c_int64), C.c_char_p, C.c_int32]),
     "edenhip_kernel_count": (C.c_int32, [C.c_void_p]),
     "edenhip_get_kernel_info": (C.c_int, [C.c_void_p, C.c_int32, C.POINTER(KernelInfo)]),
+    "edenhip_get_kernel_symbol": (C.c_int, [C.c_void_p, C.c_int32, C.c_char_p, C.c_int32]),
     "edenhip_get_kernel_cells": (C.c_int, [C.c_void_p, C.c_int32, _P, C.c_int32]),
     "edenhip_adj_create": (C.c_int, [C.POINTER(ModelDesc), C.POINTER(AdjOptions), C.POINTER(C.c_void_p)]),
     "edenhip_adj_sizes": (C.c_int, [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_int64), C.POINTER(C.c_int64),

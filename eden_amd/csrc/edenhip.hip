@@ -84,9 +84,9 @@ struct Bucket {
     int64_t lean_bytes = 0;   // its largest cell's LDS there
     bool gates_lds = true;    // the general kernel's gate table is in LDS, else in global memory
     bool long_lists = false;  // a compartment with SYN_MANY synapses or more
+    int form(bool net) const { return tpb + (gates_lds ? 0 : 1) + (net && long_lists ? 2 : 0); }
     const void *kernel(bool net) const {
-        const int form = tpb + (gates_lds ? 0 : 1) + (net && long_lists ? 2 : 0);
-        return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(form, split, net);
+        return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(form(net), split, net);
     }
     std::vector<int32_t> order;    // tree-cell indices, largest first
     int32_t nmax = 0;
@@ -2490,6 +2490,25 @@ int edenhip_get_kernel_info(const edenhip_ctx *ctx, int32_t i, edenhip_kernel_in
     out->n_comps = b.comps;
     out->launches = b.launches;
     out->total_ms = b.ms;
+    return 0;
+}
+
+int edenhip_get_kernel_symbol(const edenhip_ctx *ctx, int32_t i, char *symbol, int32_t len) {
+    edenhip_kernel_info k;
+    if (!symbol || len <= 0 || edenhip_get_kernel_info(ctx, i, &k) != 0) return EDENHIP_E_INVALID;
+    const int32_t b = i - (ctx->n_point > 0 ? 1 : 0);
+    if (b >= 0) {
+        const Bucket &bk = ctx->buckets[(size_t)b];
+        const char *split = bk.split ? "true" : "false";
+        if (bk.lean)
+            std::snprintf(k.name, sizeof(k.name), "lean_tree_kernel<%d, %s>", bk.tpb, split);
+        else
+            std::snprintf(k.name, sizeof(k.name), "tree_kernel<%d, %s, %s>", bk.form(ctx->tree_net), split,
+                          ctx->tree_net ? "true" : "false");
+    } else if (ctx->netwin && ctx->net_quad) {
+        std::snprintf(k.name, sizeof(k.name), "net_quad_kernel<%d>", ctx->net_groups);
+    }
+    std::snprintf(symbol, (size_t)len, "%s", k.name);
     return 0;
 }
 

@@ -465,16 +465,19 @@ class Simulation:
         return ms.value, nl.value, name.value.decode()
 
     def kernel_infos(self):
-        """Per-kernel launch statistics: list of dicts (name, threads_per_block, grid, cells,
-        comps, lds_bytes, launches, total_ms, cell_index array)."""
+        """Per-kernel launch statistics: list of dicts (name: the launch shape, symbol: the kernel
+        as a profiler lists it, threads_per_block, grid, cells, comps, lds_bytes, launches,
+        total_ms, cell_index array)."""
         out = []
         for i in range(self.lib.edenhip_kernel_count(self.h)):
             ki = N.KernelInfo()
             self._check(self.lib.edenhip_get_kernel_info(self.h, i, C.byref(ki)), "get_kernel_info")
             cells = np.empty(max(1, ki.n_cells), np.int32)
             self._check(self.lib.edenhip_get_kernel_cells(self.h, i, N.ptr(cells), len(cells)), "get_kernel_cells")
-            out.append(dict(name=ki.name.decode(), threads_per_block=ki.threads_per_block, grid=ki.grid,
-                            cells=ki.n_cells, comps=ki.n_comps, lds_bytes=ki.lds_bytes, launches=ki.launches,
+            symbol = C.create_string_buffer(64)
+            self._check(self.lib.edenhip_get_kernel_symbol(self.h, i, symbol, 64), "get_kernel_symbol")
+            out.append(dict(name=ki.name.decode(), symbol=symbol.value.decode(),
+                            threads_per_block=ki.threads_per_block, grid=ki.grid, cells=ki.n_cells, comps=ki.n_comps, lds_bytes=ki.lds_bytes, launches=ki.launches,
                             total_ms=ki.total_ms,
                             cell_index=cells[: ki.n_cells]))
         return out

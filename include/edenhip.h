@@ -425,9 +425,9 @@ int edenhip_kernel_stats(const edenhip_ctx *ctx, double *total_ms, int64_t *laun
  * the chunks run since create or reset, the time from the event recorded before the
  * kernel's first launch in a chunk to the event after its last, on the kernel's stream. */
 typedef struct edenhip_kernel_info {
-    char name[64];               /* kernel name as a profiler lists it, without arguments (tree
-                                    cells: always the general kernel's, also where
-                                    lean_tree_kernel runs them) */
+    char name[64];               /* the kernel's launch shape; tree cells:
+                                    tree_kernel<threads, channel wave, network>, whichever kernel
+                                    runs them (edenhip_get_kernel_symbol) */
     int32_t threads_per_block;
     int32_t grid;                /* workgroups per launch */
     int32_t n_cells;             /* cells this kernel advances */
@@ -439,6 +439,9 @@ typedef struct edenhip_kernel_info {
 
 int32_t edenhip_kernel_count(const edenhip_ctx *ctx);
 int edenhip_get_kernel_info(const edenhip_ctx *ctx, int32_t i, edenhip_kernel_info *out);
+/* Kernel i as a profiler lists it, without arguments: lean_tree_kernel<...> for passive trees on
+ * active somata, else tree_kernel<threads + form, ...>, or the point kernel. Cut to len. */
+int edenhip_get_kernel_symbol(const edenhip_ctx *ctx, int32_t i, char *symbol, int32_t len);
 /* Descriptor cell indices advanced by kernel i (n_cells of them), in work-queue order. */
 int edenhip_get_kernel_cells(const edenhip_ctx *ctx, int32_t i, int32_t *cells, int32_t max_cells);
 
