@@ -2107,8 +2107,14 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
         }
         return 0;
     };
+    // windows of the general network path (initial steps, and step 0, are launches of one)
+    auto count_windows = [&](int64_t a, int64_t b) {
+        const int64_t W = ctx->step_window, n = b - std::max<int64_t>(a, 1);
+        if (W > 1 && n > 0) ctx->net_windows += (n + W - 1) / W;
+    };
     if (!graph) {
         TRY(issue(s0, s1, prof));
+        count_windows(s0, s1);
     } else {
         // per-step launches captured in graphs of up to 256 steps (kernels only: the kernels
         // reset their own work queues, nothing is cleared with a memset node), kept for the
@@ -2139,6 +2145,7 @@ static int launch_chunk(edenhip_ctx *ctx, int64_t s0, int64_t s1, int64_t row0) 
                 ctx->graphs.push_back({a, b, row0, exec, nl - nl0});
             }
             HIPCHECK(ctx, hipGraphLaunch(exec, ctx->stream));
+            count_windows(a, b);
         }
     }
     if (graph && ctx->opt.profile) {
@@ -2528,7 +2535,7 @@ int edenhip_get_kernel_cells(const edenhip_ctx *ctx, int32_t i, int32_t *cells, 
 int edenhip_network_stats(edenhip_ctx *ctx, int32_t *window_steps, int64_t *windows, int64_t *windows_rerun,
                           int64_t *synaptic_events) {
     if (!ctx) return EDENHIP_E_INVALID;
-    if (window_steps) *window_steps = ctx->netwin ? ctx->net_W : 1;
+    if (window_steps) *window_steps = ctx->netwin ? ctx->net_W : ctx->step_window;
     if (windows) *windows = ctx->net_windows;
     if (windows_rerun) *windows_rerun = ctx->net_redone;
     if (synaptic_events) {

@@ -477,7 +477,8 @@ class Simulation:
             symbol = C.create_string_buffer(64)
             self._check(self.lib.edenhip_get_kernel_symbol(self.h, i, symbol, 64), "get_kernel_symbol")
             out.append(dict(name=ki.name.decode(), symbol=symbol.value.decode(),
-                            threads_per_block=ki.threads_per_block, grid=ki.grid, cells=ki.n_cells, comps=ki.n_comps, lds_bytes=ki.lds_bytes, launches=ki.launches,
+                            threads_per_block=ki.threads_per_block, grid=ki.grid, cells=ki.n_cells,
+                            comps=ki.n_comps, lds_bytes=ki.lds_bytes, launches=ki.launches,
                             total_ms=ki.total_ms,
                             cell_index=cells[: ki.n_cells]))
         return out

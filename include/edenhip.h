@@ -446,8 +446,9 @@ int edenhip_get_kernel_symbol(const edenhip_ctx *ctx, int32_t i, char *symbol, i
 int edenhip_get_kernel_cells(const edenhip_ctx *ctx, int32_t i, int32_t *cells, int32_t max_cells);
 
 /* Network path figures since create or reset: steps per window (1 = one launch per step),
- * windows run, windows run again step by step (see edenhip_options.network_window), and
- * spike-triggered synaptic events received (-1 when not counted: per-step path). */
+ * windows run, windows run again step by step (networks of one-compartment cells, see
+ * edenhip_options.network_window), and spike-triggered synaptic events received (there only, else
+ * -1: not counted). */
 int edenhip_network_stats(edenhip_ctx *ctx, int32_t *window_steps, int64_t *windows, int64_t *windows_rerun,
                           int64_t *synaptic_events);
 
