@@ -135,6 +135,7 @@ EXPORTS = {
     "edenhip_write_events": (C.c_int, [C.c_char_p, C.c_int, C.c_int32, _P, _P, _P, C.c_int64, _P, C.c_int64]),
     "edenhip_format_number": (C.c_int, [C.c_double, C.c_char_p, C.c_int32]),
     "edenhip_diag_divide": (C.c_int, [C.c_uint64, C.c_int64, _P, C.c_int32, C.POINTER(C.c_int64)]),
+    "edenhip_diag_reciprocals": (C.c_int, [C.c_uint64, C.c_int64, _P, C.c_int32, C.POINTER(C.c_int64)]),
     "edenhip_network_stats": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_int64),
                                         C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
     "edenhip_size_limits": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32)]),

@@ -167,13 +167,14 @@ struct LemsCellArgs {
 // the compiler's division takes eleven.
 __device__ __forceinline__ float div_c(float n, double r) { return (float)((double)n * r); }
 
-// The same for every finite n, denormal quotients included: 1 / d as the sum of two doubles, so
-// that the product is within 2^-104 of n / d before it is rounded, and a quotient in the middle
-// of two denormals comes out exactly and is then rounded to even as n / d is.
+// The same for every finite n and non-zero d, denormal quotients included: 1 / d as the sum of two
+// doubles, so that the product is within 2^-104 of n / d before it is rounded, and a quotient in
+// the middle of two denormals comes out exactly and is then rounded to even as n / d is. (A zero
+// may come out with the other sign.)
 struct Recip2 {
     double hi, lo;
 };
-__device__ __forceinline__ Recip2 recip2(float d) {
+__host__ __device__ __forceinline__ Recip2 recip2(float d) {
     Recip2 r;
     r.hi = 1.0 / (double)d;
     r.lo = fma(-r.hi, (double)d, 1.0) / (double)d;

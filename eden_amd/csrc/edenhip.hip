@@ -1781,13 +1781,7 @@ static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std
             for (float x : {st.tau_rise, st.tau_decay}) ok = ok && x > 0x1p-20f && x < 0x1p40f;
             if (K.n == NET_CLASSES) { ok = false; break; }
             const int c = K.n++;
-            auto recip = [](float x, double &hi, double &lo) {   // recip2
-                hi = 1.0 / (double)x;
-                lo = std::fma(-hi, (double)x, 1.0) / (double)x;
-            };
-            K.c[c] = NetClass{st.gbase, st.erev, jump, t, 0, 0, 0, 0};
-            recip(st.tau_rise, K.c[c].rise_hi, K.c[c].rise_lo);
-            recip(st.tau_decay, K.c[c].decay_hi, K.c[c].decay_lo);
+            K.c[c] = NetClass{st.gbase, st.erev, jump, t, recip2(st.tau_rise), recip2(st.tau_decay)};
         }
         int groups = 0;
         for (size_t b0 = 0; b0 < point.size() && ok; b0 += 16) {

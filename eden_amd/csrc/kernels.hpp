@@ -121,7 +121,7 @@ constexpr int NET_CLASSES = 4;
 struct alignas(16) NetClass {
     float gbase, erev, jump;       // jump: weight property * waveform factor
     int32_t type;
-    double rise_hi, rise_lo, decay_hi, decay_lo;   // recip2 of the time constants
+    Recip2 rise, decay;            // of the time constants
 };
 struct NetClasses {
     int32_t n;                     // types in use, at most NET_CLASSES

@@ -435,8 +435,8 @@ net_quad_kernel(DevTables T, NetTables Nt, const DGate *__restrict__ gates_g, Ne
                     float An[4], Bn[4];
 #pragma unroll
                     for (int u = 0; u < 4; u++) {
-                        An[u] = A[i][u] + dt * div_c2(-A[i][u], Recip2{K.rise_hi, K.rise_lo});
-                        Bn[u] = B[i][u] + dt * div_c2(-B[i][u], Recip2{K.decay_hi, K.decay_lo});
+                        An[u] = A[i][u] + dt * div_c2(-A[i][u], K.rise);
+                        Bn[u] = B[i][u] + dt * div_c2(-B[i][u], K.decay);
                     }
                     if ((ev_any >> (4 * i)) & 15) {
 #pragma unroll
@@ -468,8 +468,8 @@ net_quad_kernel(DevTables T, NetTables Nt, const DGate *__restrict__ gates_g, Ne
                 const bool fired = init || pt > pi;
                 const float a = pA, b = pB;
                 pt = pt + dt * 1.0f;
-                pA = a + dt * div_c2(-a, Recip2{K.rise_hi, K.rise_lo});
-                pB = b + dt * div_c2(-b, Recip2{K.decay_hi, K.decay_lo});
+                pA = a + dt * div_c2(-a, K.rise);
+                pB = b + dt * div_c2(-b, K.decay);
                 if (fired) {
                     // (addresses formed here, not kept for the window)
                     int32_t p = pb + qs, gc = (int32_t)g;
