@@ -1088,18 +1088,22 @@ int build_adj(edenhip_adj *a, const edenhip_model_desc *d) {
         nmax = std::max(nmax, n);
     }
     // workgroup size: lanes for a cell's compartments and for pairs of its gates, beside the wave
-    // that solves
+    // that solves (a gradient of 100 steps, 64 / 128 / 256 threads: 64 cells of 100 compartments 3.3 / 2.2
+    // / 1.8 ms, 256 of 64 2.6 / 1.8 / 1.7, 2,000 of 100 10.2 / 6.7 / 5.0, 2,000 of 30 2.3 / 2.0 / 2.9)
+    int64_t most_gates = 0;
     for (int c = 0; c < d->n_cells; c++) {
         const int64_t c0 = d->cell_comp_begin[c], c1 = d->cell_comp_begin[c + 1];
         int64_t ngate = 0;
         for (int64_t ch = d->comp_chan_begin[c0]; ch < d->comp_chan_begin[c1]; ch++)
             ngate += d->channel_types[d->chan_type[ch]].n_gates;
+        most_gates = std::max(most_gates, ngate);
         const int64_t want = std::max<int64_t>(c1 - c0, ngate / 2);
         tpb = std::max(tpb, want > 64 ? 256 : 128);
     }
     tpb = std::min(tpb, 256);
     // opt overrides applied by the caller
-    a->tpb = a->tpb > 0 ? a->tpb : tpb;
+    const bool by_rule = a->tpb <= 0;
+    if (by_rule) a->tpb = tpb;
     for (int c = 0; c < d->n_cells; c++) {
         const int64_t c0 = d->cell_comp_begin[c], c1 = d->cell_comp_begin[c + 1];
         const int32_t n = (int32_t)(c1 - c0);
@@ -1186,6 +1190,17 @@ int build_adj(edenhip_adj *a, const edenhip_model_desc *d) {
         char msg[160];
         std::snprintf(msg, sizeof msg, "cell too large for the adjoint kernels' LDS (%zu bytes needed, 163,840 available)", a->lds);
         return afail(a, EDENHIP_E_LIMIT, msg);
+    }
+    // one wave a cell where a pass of it takes all gates and two waves a cell are more than the chip
+    // holds at once, so that the second one would wait for a place instead of hiding anything (64 and
+    // 128 threads, cells of 10 compartments: 2,000 cells 1.6 and 1.5 ms, 2,500 1.8 and 2.2, 16,000 6.2
+    // and 8.1; of 22, 66 gates: 4,000 cells 3.8 and 3.3)
+    if (by_rule && a->tpb == 128 && most_gates <= 64) {
+        int cus = 0, f = 0, b = 0;
+        AHIP(a, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, a->device));
+        AHIP(a, hipOccupancyMaxActiveBlocksPerMultiprocessor(&f, fwd_kernel(128), 128, a->lds));
+        AHIP(a, hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, bwd_kernel(128), 128, a->lds));
+        if ((int64_t)d->n_cells > (int64_t)std::min(f, b) * cus) a->tpb = 64;
     }
     a->K = std::max(1, a->K);
     const int64_t steps = a->rows;   // steps 1..rows-1 are differentiated

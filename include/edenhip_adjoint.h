@@ -51,7 +51,7 @@ typedef struct edenhip_adj edenhip_adj;
 
 typedef struct edenhip_adj_options {
     int32_t checkpoint_steps;    /* steps between checkpoints (0 = 500) */
-    int32_t threads_per_cell;    /* 0 = by cell size, or 64/128/256 */
+    int32_t threads_per_cell;    /* 0 = by cell size and number, or 64/128/256 */
     int32_t device;
     int32_t store_states;        /* 0 = keep every step's state in device memory when it takes at
                                     most half of the free memory, else checkpoints and recompute;
