@@ -1622,9 +1622,10 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     // several buckets on the main one, before its bucket, as a fourth stream to fork and join in
     // every step costs more than it hides (201 steps with 20 point cells: 48 trees of 100 to 600
     // compartments, three buckets, 13.6 -> 12.0 ms; 100 of 700 to 1,900, two, 13.9 -> 12.6; one
-    // bucket of 1,024 trees 14.6 beside it, 15.0 before it)
+    // bucket of 1,024 trees 14.6 beside it, 15.0 before it). In a captured graph the streams are only
+    // an order of nodes, and a branch of their own is faster (the first of these 7.5 ms, 9.0 without)
     ctx->point_stream = ctx->stream;
-    const bool single = (ctx->network || ctx->opt.persistent < 0) && window_len == 1;
+    const bool single = (ctx->network || ctx->opt.persistent < 0) && window_len == 1 && !ctx->opt.use_graph;
     if (ctx->n_point > 0 && !ctx->buckets.empty() && ctx->buckets.size() < (single ? 2u : 4u)) {
         TRY(pool_stream(ctx, (int)ctx->buckets.size(), &ctx->point_stream));
         HIPCHECK(ctx, hipEventCreateWithFlags(&ctx->point_done, hipEventDisableTiming));
