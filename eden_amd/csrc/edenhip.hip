@@ -52,9 +52,9 @@ bool const_below_root(const edenhip_model_desc *d, int64_t c0, int32_t n) {
 
 // Voltages at which gate_next_fast's divisions stay inside the normal floats: rate parameters of
 // moderate size (any other gate gets the empty range, so the general path), and a voltage within
-// 24 scales of each midpoint. The exponentials are then within 2^+-35, every rate within
+// 23.9 scales of each midpoint. The exponentials are then within 2^+-35, every rate within
 // 2^-63 .. 2^58 (or zero), inf above 2^-121 and the time factor within 2^+-84. HH squid rates
-// (scale 10 around -40 mV): -279 .. 173 mV.
+// (m: scale 10 around -40 mV): -279 .. 199 mV.
 void gate_safe_range(DGate &G, float dt) {
     G.ras = 1.0 / (double)G.as;
     G.rbs = 1.0 / (double)G.bs;
@@ -122,7 +122,7 @@ struct edenhip_ctx {
     float dt = 0;
     int64_t NC = 0, n_poi = 0, n_slots = 0, total_rows = 0, rows_done = 0, next_step = -3;
     int n_cells = 0;
-    bool network = false;      // spike recipients: one launch per step
+    bool network = false;      // spike recipients or kernels between the steps: windows, or one step a launch
     bool tree_net = false;     // tree kernels of the NET form (network, or synapses on tree cells)
     bool point_quad = false;   // point cells run four lanes per cell (no synapses, inputs, spikes)
     // host mirrors for output mapping
@@ -1604,7 +1604,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         // out of wave slots first and the extra wave per cell costs more than it hides. For
         // 2 and 4 cable waves the extra wave costs a workgroup per CU, which those sizes
         // need more.
-        // Networks run one step per launch with the NET kernels, which have no channel wave.
+        // Networks run the NET kernels, which have no channel wave.
         // channel_wave overrides the rule per workgroup size
         const int cw = ctx->opt.channel_wave[b.tpb == 64 ? 0 : b.tpb == 128 ? 1 : b.tpb == 256 ? 2 : 3];
         const bool rule = b.tpb == 512 || (b.tpb == 64 && (int64_t)bc.size() <= 4 * (int64_t)ctx->n_cu);
@@ -1838,8 +1838,10 @@ static int build_netwin(edenhip_ctx *ctx, const edenhip_model_desc *d, const std
     }
     if (ctx->net_quad) TRY(upload(ctx, &ctx->d_net_rare, std::vector<NetRare>(1, NetRare{ctx->T})));
     // The one case a window cannot decide, a pending arrival that lies in two consecutive step
-    // windows [t, t + dt), needs windows that overlap. Where the float times do not, as with any
-    // dt of whole microseconds, no window has to be checked against step order.
+    // windows [t, t + dt), needs windows that overlap. Where no two of the run do, no window has to be
+    // checked against step order. Float times of whole microseconds are exact up to 16.8 s; with
+    // steps of 25 us windows are disjoint up to 134 s, with 3, 7 or 11 us up to 16.8 s, and a run that
+    // goes on beyond is checked from its start.
     ctx->net_free = !ctx->steps_overlap && ctx->opt.network_window != -2;
     ctx->net_W = W;
     ctx->net_cur = 0;

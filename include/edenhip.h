@@ -185,7 +185,8 @@ typedef struct edenhip_lems_synapses {
  * beside lems_syn (eden_amd.lems_cells emits it). A point-neuron cell has one compartment,
  * without channels or Poisson inputs; its synapses take the generic path (lems), and the
  * compartment's V mirrors the type's membrane-voltage state variable (its synapses' and gap
- * junction peers' voltage). Models with point neurons run one launch per step. */
+ * junction peers' voltage). Where only point neurons have generic synapses, none of them a peer,
+ * a launch runs several steps as far as the delays allow, else one. */
 typedef struct edenhip_lems_cells {
     int32_t n_types;
     const char *source;           /* HIP C++ source, NUL-terminated */
@@ -279,7 +280,8 @@ typedef struct edenhip_model_desc {
      * its j-th gate variable (its channel distributions in order, each type's gates in order),
      * as an OutputColumn of a channel gate's q records it; for a point neuron (abi_version >= 4)
      * j >= 0 is its j-th state variable and -1 its membrane-voltage state variable. NULL = V
-     * everywhere. A model that records gate variables runs one launch per step. */
+     * everywhere. A model that records gate variables runs one launch per step; point
+     * neurons' state variables alone do not ask for that. */
     const int32_t *record_gate;
 
     /* (abi_version >= 4) LEMS point neurons, or NULL */
