@@ -32,7 +32,7 @@ from .model import Simulation
 DEFAULT = (256, 512, 1024, 2047)
 # candidate values per movable limit (each at most 4 compartments per thread)
 CANDIDATES = ((128, 192, 256), (384, 448, 512), (768, 896, 1024))
-# the same in a network, whose own limits are 64, 128, 512 or 256, 512, 512
+# the same in a network, whose own limits are 64, 128, 512 or 256, 512, 512 (or 1024)
 NETWORK_CANDIDATES = ((64, 128, 256), (128, 256, 512), (512, 768, 1024))
 
 

@@ -973,17 +973,20 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
     // 1.9 ms, 48 of 100 to 600 3.3 -> 2.7, 256 active ones of 60 to 250 4.9 -> 3.8, 1,024 of 20 to 150
     // 3.1 -> 2.8; slower only for 600 of 700 to 1,500, 4.1 -> 5.4; without synapses more lanes are
     // slower, 256 active trees of 60 to 160 14.5 -> 21 ms). With launches of one step every size in
-    // use is a launch of its own, forked and joined in each step, so the limits leave few sizes
-    // (256 / 512 / 1024, 64 / 128 / 512 and 256 / 512 / 512: 48 trees of 20 to 150 compartments 7.9,
-    // 13.5 and 7.9 ms, 100 of 700 to 1,900 13.9, 11.1 and 11.1, 48 with generic synapses 8.2, 11.2
-    // and 8.2)
+    // use is a launch of its own, forked and joined in each step, so the limits leave few sizes: up to
+    // 256 compartments a wave (256 / 512 / 1024 and 64 / 128 / 512: 48 trees of 20 to 150 compartments
+    // 7.9 and 13.5 ms, with generic synapses 8.2 and 11.2), and where a cell of more than 1,024 needs
+    // 512 threads anyway, those of more than 512 with it (256 / 512 / 1024 and 256 / 512 / 512: 1,000
+    // trees of 600 to 1,800 13.4 and 10.8 ms; of 300 to 1,000, the same number of sizes, 9.3 and 12.1)
     int32_t *const limits = ctx->limits;
     std::copy(ctx->opt.size_limits, ctx->opt.size_limits + 4, limits);
     if (limits[0] == 0 && limits[1] == 0 && limits[2] == 0 && limits[3] == 0) {
         const bool net = d->comp_spike_begin[NC] > 0;
         limits[0] = net && window_len > 1 ? 64 : 256;
         limits[1] = net && window_len > 1 ? 128 : 512;
-        limits[2] = net ? 512 : 1024;
+        bool over_1024 = false;
+        for (int c = 0; c < d->n_cells; c++) over_1024 = over_1024 || d->cell_comp_begin[c + 1] - d->cell_comp_begin[c] > 1024;
+        limits[2] = net && (window_len > 1 || over_1024) ? 512 : 1024;
         limits[3] = MAX_TREE_N;
     }
     {

@@ -334,7 +334,8 @@ typedef struct edenhip_options {
     int32_t size_limits[4];       /* largest tree cell (compartments) given 64, 128, 256 and
                                      512 threads; all 0 = 256, 512, 1024, 2047, or in a
                                      network of tree cells 64, 128, 512, 2047 where launches run
-                                     several steps and 256, 512, 512, 2047 where they run one.
+                                     several steps, and 256, 512, 512, 2047 where they run one
+                                     and a cell has more than 1,024 compartments.
                                      A cell takes the first size whose limit holds it (each limit at most 4
                                      compartments per thread; the 512 limit must be 2047).
                                      eden_amd.autotune picks them by timing short runs. */

@@ -53,3 +53,12 @@ def test_autotuner_starts_from_the_networks_limits():
     with Simulation(m) as a, Simulation(m, size_limits=limits) as b:
         assert a.size_limits() == WINDOW and b.size_limits() == limits
         assert np.array_equal(a.run_all(), b.run_all())
+
+
+@pytest.mark.parametrize("largest,limits", [(1024, (256, 512, 1024, 2047)), (1025, SINGLE)])
+def test_single_steps_share_the_largest_size_where_a_cell_needs_it(largest, limits):
+    m = configs.mixed_network(tree_sizes=(40, 600, largest), n_point=2, n_conn=30, t_final_ms=2.0, delay_ms=(0.025, 0.05))
+    with Simulation(m) as sim:
+        assert sim.size_limits() == limits
+        tr = sim.run_all()
+    assert np.array_equal(tr, oracle.run(m)[0])
