@@ -85,7 +85,10 @@ struct Bucket {
     int64_t lean_bytes = 0;   // its largest cell's LDS there
     bool gates_lds = true;    // the general kernel's gate table is in LDS, else in global memory
     bool long_lists = false;  // a compartment with SYN_MANY synapses or more
-    int form(bool net) const { return tpb + (gates_lds ? 0 : 1) + (net && long_lists ? 2 : 0); }
+    bool single = false;      // its launches are of one step
+    int form(bool net) const {
+        return tpb + (gates_lds ? 0 : 1) + (net && long_lists ? 2 : 0) + (net && long_lists && single && tpb == 64 ? 4 : 0);
+    }
     const void *kernel(bool net) const {
         return lean ? lean_tree_kernel_ptr(tpb, split) : tree_kernel_ptr(form(net), split, net);
     }
@@ -1612,6 +1615,7 @@ static int build(edenhip_ctx *ctx, const edenhip_model_desc *d) {
         const int cw = ctx->opt.channel_wave[b.tpb == 64 ? 0 : b.tpb == 128 ? 1 : b.tpb == 256 ? 2 : 3];
         const bool rule = b.tpb == 512 || (b.tpb == 64 && (int64_t)bc.size() <= 4 * (int64_t)ctx->n_cu);
         b.split = (cw > 0 || (cw == 0 && rule)) && ctx->opt.persistent >= 0 && !ctx->tree_net;
+        b.single = ctx->tree_net && window_len == 1;
         // lean_tree_kernel runs every bucket of lean cells, also where its blocks, twice the LDS,
         // leave fewer cells in flight (481 rows of 4,096 cells of up to 400 compartments 5.3 -> 3.4
         // ms, of up to 2,000 11.5 -> 8.4; with tree_kernel for the 512-thread bucket alone 9.0)

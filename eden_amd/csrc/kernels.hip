@@ -240,13 +240,20 @@ __device__ __forceinline__ void channel_phase(const DGate *gates, const uint32_t
 // the point kernel does, and a compartment with spike recipients sends its spikes to the
 // next step's flags; both are complex compartments, so the per-slot code of the other
 // compartments is unchanged and the NET = false kernels carry none of it.
-// FORM: the cable group's threads; two more where a compartment's synapses are read eight at a time
-// (a bucket with a long list, SYN_MANY), else two; one more where the gate table, up to 16 KiB, is
-// read from global memory. That is for the largest cells, whose other tables leave no room for it: a binary tree with
-// HH channels on every compartment, in a model of 64 channel types, takes up to 1,743 compartments
-// with the table in LDS and 1,937 without.
+// FORM: the cable group's threads, and
+//   1 more where the gate table, up to 16 KiB, is read from global memory. That is for the largest
+//     cells, whose other tables leave no room for it: a binary tree with HH channels on every
+//     compartment, in a model of 64 channel types, takes up to 1,743 compartments with the table in
+//     LDS and 1,937 without.
+//   2 more where a compartment's synapses are read eight at a time (a bucket with a long list,
+//     SYN_MANY), else two.
+//   4 more where such a bucket's launches are of one step: compiled for two waves a SIMD, a launch
+//     loads and stores no spilled registers (600 trees of 20 to 300 compartments with 50 synapses on
+//     each soma 17.7 -> 17.1 ms, 4,000 of 20 to 100 with 30 23.0 -> 16.5). With windows it leaves too few
+//     cells in flight (2,000 of 20 to 150 with 20 2.8 -> 3.4 ms), and so it does beyond 64 threads (500
+//     of 100 to 600 with 40 9.6 -> 10.2).
 template <int FORM, bool SPLIT, bool NET>
-__global__ void __launch_bounds__((FORM & ~3) + (SPLIT ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__((FORM & ~7) + (SPLIT ? 64 : 0)) __attribute__((amdgpu_waves_per_eu((FORM & 4) ? 2 : 4)))
 tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const DSynType *__restrict__ stypes_g,
             int n_stypes, const TreeCell *__restrict__ cells, const int32_t *__restrict__ task_order, int32_t n_tasks,
             int32_t *__restrict__ queue, const uint32_t *__restrict__ words_g, const int32_t *__restrict__ pos_g,
@@ -255,7 +262,7 @@ tree_kernel(DevTables T, const DGate *__restrict__ gates_g, int n_gates, const D
             const uint32_t *__restrict__ cflag_g, const TreeComplex *__restrict__ cx_g, int32_t cxmax_lds, int32_t nmax,
             int32_t nvmax, int32_t ngmax, int32_t nctmax, int32_t ninmax, int32_t words_max, int64_t s0, int64_t s1,
             int64_t row0, float dt) {
-    constexpr int TPB = FORM & ~3;
+    constexpr int TPB = FORM & ~7;
     constexpr bool GATES_LDS = (FORM & 1) == 0;
     constexpr int K = TREE_SLOTS;
     constexpr int NT = TPB + (SPLIT ? 64 : 0);
@@ -1201,6 +1208,7 @@ static const void *tree_kernel_of(int form) {
     }
     if constexpr (NET) {
         switch (form) {
+        case 70: return reinterpret_cast<const void *>(&tree_kernel<70, SPLIT, NET>);
         case 66: return reinterpret_cast<const void *>(&tree_kernel<66, SPLIT, NET>);
         case 130: return reinterpret_cast<const void *>(&tree_kernel<130, SPLIT, NET>);
         case 258: return reinterpret_cast<const void *>(&tree_kernel<258, SPLIT, NET>);

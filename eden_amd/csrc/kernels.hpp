@@ -135,7 +135,7 @@ constexpr int NET_QUAD_MAX = 16;
 
 // form: a workgroup's threads without a channel wave (64, 128, 256, 512), plus 1 where the gate
 // table is read from global memory (256 and 512 only), plus 2 in a network where a compartment's
-// synapses are read eight at a time. net: the variant for networks (synapses on tree compartments,
+// synapses are read eight at a time, plus 4 where its launches are of one step (64 only). net: the variant for networks (synapses on tree compartments,
 // spikes sent to recipients), only without a channel wave. Null where there is none.
 const void *tree_kernel_ptr(int form, bool split, bool net);
 // Synapses of one compartment from which a bucket's kernel reads eight at a time, each a register

@@ -50,5 +50,6 @@ def test_other_kernels():
     long = dataclasses.replace(net, comp_syn_begin=at, syn_type=np.sort(net.syn_type))
     assert net.n_synapses >= 16
     assert _symbols(long) == ["point_kernel", "tree_kernel<128, false, true>", "tree_kernel<66, false, true>"]
+    assert _symbols(long, network_window=-1) == ["point_kernel", "tree_kernel<70, false, true>"]
     cells = configs.spiking_network(n_cells=40, in_degree=17, t_final_ms=3.0)
     assert _symbols(cells)[0] in ("net_quad_kernel<2>", "net_quad_kernel<4>")
